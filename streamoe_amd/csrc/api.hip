@@ -792,7 +792,7 @@ uint64_t smoe_moe_prefill_workspace_size(const smoe_expert_shape* shape, uint32_
                                          uint32_t n_experts, uint32_t k) {
   if (!shape || !shape->group || !n_tokens || !n_experts || !k) return 0;
   if (!prefill_supported(shape->hidden, shape->inter, shape->group, shape->bits, n_tokens, n_experts, k))
-    return prefill_tokens_workspace(shape->hidden, shape->inter, n_tokens, k, true);
+    return limb_prefill_workspace(shape->hidden, shape->inter, shape->group, n_tokens, n_experts, k);
   return prefill_workspace(shape->hidden, shape->inter, shape->group, n_tokens, n_experts, k, false, nullptr,
                            nullptr);
 }
@@ -819,8 +819,20 @@ int smoe_moe_prefill(smoe_handle* h, const smoe_expert_shape* shape, const void*
       !aligned(out_sum, 0, 16) || !aligned(workspace, 0, 256))
     return SMOE_ERR_MISALIGNED;
   if (!prefill_supported(shape->hidden, shape->inter, shape->group, shape->bits, n_tokens, n_experts, k)) {
-    // Shapes without grouped-GEMM tiles: one token at a time through the
-    // per-phase decode kernels.
+    // Shapes without bf16 / fp16 grouped-GEMM tiles: grouped on the int8
+    // matrix cores from three tokens on; fewer (2560 x 640, top-10: one 33 us
+    // against 48, two 65 against 49, three 96 against 57; 2048 x 512, top-8:
+    // two 35 against 41, eight 134 against 51), or a workspace too small for
+    // the grouped call, one token at a time through the per-phase decode
+    // kernels.
+    if (n_tokens > 2 &&
+        workspace_bytes >= limb_prefill_workspace(shape->hidden, shape->inter, shape->group, n_tokens, n_experts, k)) {
+      if (int rc = use_device(h)) return rc;
+      return hip_status(launch_limb_prefill(blob_geom(shape->hidden, shape->inter, shape->group, shape->bits),
+                                            (const uint8_t*)experts, stride, n_experts, idx, weights, x,
+                                            x_is_bf16 != 0, n_tokens, k, out_sum, (uint8_t*)workspace, h->err,
+                                            h->stream));
+    }
     if (workspace_bytes < prefill_tokens_workspace(shape->hidden, shape->inter, n_tokens, k, x_is_bf16 != 0))
       return SMOE_ERR_WORKSPACE_TOO_SMALL;
     if (int rc = use_device(h)) return rc;

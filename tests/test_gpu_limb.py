@@ -1,0 +1,75 @@
+"""The int8-limb GEMMs (csrc/limb.hip) at the edges of their tiles, against the
+oracle's f32 path. Bar: max|d| / max|ref| <= 1e-5. Both sides round their
+sums to f32: a sequential sum of K terms is off by about sqrt(K) 2^-24 of its
+size (5.4e-6 at 8192), the gate, up and down sums add in quadrature, and the
+limb side adds less than that."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import rel_err
+from test_gpu_prefill import _case, _torch, host
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+@pytest.mark.parametrize("name,n,H,I,E,k,bits,group,x_bf16,routing", [
+    ("one-chunk", 3, 32, 32, 4, 2, 4, 32, True, "zipf"),             # a quarter step, a quarter column block
+    ("g32-tail", 17, 96, 160, 6, 3, 3, 32, False, "hot"),            # 17 entries: an item of one row
+    ("g64-half-step", 33, 320, 192, 5, 2, 4, 64, True, "hot"),       # K = 2.5 steps, odd group counts
+    ("g128-odd", 40, 1152, 384, 9, 4, 4, 128, False, "zipf"),        # K split, 9 groups per row
+    ("g64-3bit", 48, 704, 832, 12, 6, 3, 64, True, "zipf"),          # columns not a multiple of 128
+    ("wide-g32", 7, 8160, 96, 3, 2, 3, 32, False, "zipf"),           # largest scale area
+    ("inter-2048", 5, 2080, 2016, 4, 3, 4, 32, True, "zipf"),
+    ("e1500", 20, 256, 64, 1500, 16, 4, 64, True, "zipf"),           # more experts than entries
+    ("max-entries", 1024, 64, 64, 40, 16, 4, 64, True, "zipf"),      # 16384 entries
+])
+def test_limb_prefill_matches_oracle(kernels, name, n, H, I, E, k, bits, group, x_bf16, routing):
+    got, want, _ = _case(kernels, n, H, I, E, k, bits, group, x_bf16, seed=sum(map(ord, name)), routing=routing)
+    err = rel_err(got, want)
+    print(f"limb prefill {name}: rel_err={err:.3e}")
+    assert np.all(np.isfinite(got))
+    assert err <= TOL
+
+
+def test_limb_prefill_workspace_alignment_and_nonfinite_rows(kernels):
+    """3-bit blobs at a base that is only 4-byte aligned; a workspace just
+    below the grouped call's runs token by token to the same result; a row
+    with a NaN or an infinity turns its own token's outputs into NaN and no
+    other's."""
+    import streamoe_amd as sa
+
+    torch = _torch()
+    lay = sa.ExpertLayout(320, 192, 3, 64)
+    E, n, k = 6, 19, 3
+    stride = (lay.expert_size + 15) // 16 * 16
+    buf = torch.empty(E * stride + 16, dtype=torch.uint8, device="cuda")
+    arena = buf[4:4 + E * stride]
+    assert kernels.synth_experts(arena, E, stride, lay, 77) == 0
+    idx, w = sa.zipf_routing(n, E, k, 1.1, seed=3)
+    x = torch.empty((n, 320), dtype=torch.float32, device="cuda")
+    assert kernels.synth_normal_f32(x, 78, 1.0) == 0
+    idx_d, w_d = torch.from_numpy(idx).cuda(), torch.from_numpy(w).cuda()
+    need = kernels.moe_prefill_workspace_size(lay, n, E, k)
+
+    def run(ws_bytes, rows):
+        out = torch.full((n, 320), 7.0, dtype=torch.float32, device="cuda")
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+        assert kernels.moe_prefill(lay, arena, stride, E, idx_d, w_d, rows, False, n, k, out, ws) == 0
+        kernels.sync()
+        return host(out)
+
+    got = run(need, x)
+    want = oracle.moe_permute_fuse(host(arena), stride, 3, 320, 192, 64, host(x),
+                                   oracle.build_expert_buckets(idx, w, n, k, E), n)
+    assert rel_err(got, want) <= TOL
+    assert rel_err(run(need - 256, x), want) <= TOL
+    bad = x.clone()
+    bad[4, 100] = float("nan")
+    bad[9, 319] = float("-inf")
+    out = run(need, bad)
+    rest = [t for t in range(n) if t not in (4, 9)]
+    assert np.all(np.isnan(out[[4, 9]]))
+    assert np.array_equal(out[rest], got[rest])
