@@ -183,9 +183,13 @@ uint64_t smoe_qmm_workspace_size(uint32_t in_dim, uint32_t group, uint32_t n_tok
  * N > 1). The GEMM takes bits 4 or 3, group 32/64/128, in_dim a
  * multiple of 256 (<= 16384), out_dim a multiple of 256; weights, scales,
  * biases, x, y 16-byte aligned, biases after the scales; workspace
- * 256-byte aligned. Other shapes with in_dim <= 8192 (a multiple of the
- * group) run smoe_qmv's kernel once per token row (x rows 16-byte
- * aligned; workspace unused). Enqueue-only, allocates nothing. */
+ * 256-byte aligned. Few rows, small products and the other shapes with
+ * in_dim <= 8192 (a multiple of the group; x rows 16-byte aligned) run on
+ * int8 MFMA over the rows as 31-bit block floating point (f32 precision; a
+ * row with a NaN or an infinity gives a row of NaN). For those other
+ * shapes, one row, 8-bit weights and a workspace smaller than
+ * smoe_qmm_workspace_size or not 256-byte aligned run smoe_qmv's kernel
+ * once per row. Enqueue-only, allocates nothing. */
 int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, uint32_t out_dim,
              uint32_t in_dim, uint32_t n_tokens, void* workspace, uint64_t workspace_bytes);
 

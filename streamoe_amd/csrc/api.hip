@@ -270,7 +270,9 @@ int smoe_qmv(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
 
 uint64_t smoe_qmm_workspace_size(uint32_t in_dim, uint32_t group, uint32_t n_tokens) {
   if (!in_dim || !group || !n_tokens) return 0;
-  return qmm_workspace(in_dim, group, n_tokens, nullptr, nullptr);
+  const uint64_t tiles = qmm_workspace(in_dim, group, n_tokens, nullptr, nullptr);
+  const uint64_t limbs = limb_qmm_workspace(in_dim, group, n_tokens);
+  return tiles > limbs ? tiles : limbs;
 }
 
 int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, uint32_t out_dim,
@@ -278,12 +280,16 @@ int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
   if (!h || !x || !y || !out_dim || !n_tokens || !workspace) return SMOE_ERR_INVALID_ARG;
   QView v;
   if (int rc = qview(w, in_dim, &v, true)) return rc;
+  const bool limb_ws = aligned(workspace, 0, 256) && workspace_bytes >= limb_qmm_workspace(in_dim, w->group_size, n_tokens);
   if (!qmm_supported(in_dim, out_dim, w->group_size, w->bits, n_tokens)) {
-    // Shapes without GEMM tiles (in_dim or out_dim not a multiple of 256,
-    // in_dim up to 8192): one k_qmv per token row, as smoe_qmv computes it.
+    // Shapes without bf16 GEMM tiles (in_dim or out_dim not a multiple of
+    // 256, in_dim up to 8192): the limb GEMM; one row, 8-bit weights or a
+    // small workspace: one k_qmv per token row, as smoe_qmv computes it.
     if (in_dim > 8192) return SMOE_ERR_UNSUPPORTED_SHAPE;
     if (!aligned(x, 0, 16)) return SMOE_ERR_MISALIGNED;
     if (int rc = use_device(h)) return rc;
+    if (n_tokens > 1 && w->bits != 8 && limb_ws)
+      return hip_status(launch_limb_qmm(v, x, y, out_dim, in_dim, n_tokens, (uint8_t*)workspace, h->stream));
     for (uint32_t t = 0; t < n_tokens; ++t) {
       bool unsupported = false;
       const hipError_t e = launch_qmv(v, x + (size_t)t * in_dim, y + (size_t)t * out_dim, out_dim, in_dim,
@@ -304,6 +310,13 @@ int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
   if (workspace_bytes < qmm_workspace(in_dim, w->group_size, n_tokens, nullptr, nullptr))
     return SMOE_ERR_WORKSPACE_TOO_SMALL;
   if (int rc = use_device(h)) return rc;
+  if (n_tokens == 1 && in_dim <= 8192) {  // 2048 -> 4096: 5 us, the limb GEMM 10, k_pf_mm 130
+    bool unsupported = false;
+    const hipError_t e = launch_qmv(v, x, y, out_dim, in_dim, h->stream, &unsupported);
+    if (!unsupported) return hip_status(e);
+  }
+  if (limb_ws && limb_qmm_faster(out_dim, in_dim, n_tokens))
+    return hip_status(launch_limb_qmm(v, x, y, out_dim, in_dim, n_tokens, (uint8_t*)workspace, h->stream));
   PfArgs a{};
   qmm_workspace(in_dim, w->group_size, n_tokens, &a, (uint8_t*)workspace);
   a.g.bits = w->bits;

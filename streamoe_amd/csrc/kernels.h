@@ -202,6 +202,12 @@ uint64_t limb_prefill_workspace(uint32_t hidden, uint32_t inter, uint32_t group,
 hipError_t launch_limb_prefill(const BlobGeom& g, const uint8_t* experts, uint64_t stride, uint32_t E,
                                const int32_t* idx, const float* w, const void* x, bool x_bf16, uint32_t n, uint32_t k,
                                float* out, uint8_t* ws, uint32_t* err, hipStream_t st);
+// Dense matmul on the same kernel (4- and 3-bit, in_dim a multiple of 32 up
+// to 8192).
+uint64_t limb_qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens);
+bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t n);
+hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,
+                           uint8_t* ws, hipStream_t st);
 bool prefill_supported(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t bits,
                        uint32_t n_tokens, uint32_t n_experts, uint32_t k);
 hipError_t launch_prefill(const PfArgs& a, uint32_t n_cu, hipStream_t st);

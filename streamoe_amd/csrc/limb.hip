@@ -21,8 +21,6 @@
 // term sum_g b_g sum_{j in g} x_j runs on v_mfma_f32_16x16x4_f32 over the
 // group sums (scaled by 2^f), and the result is acc 2^-f. A row with an
 // infinity or NaN gets NaN group sums, so all its outputs are NaN.
-#include <type_traits>
-
 #include "common.h"
 #include "kernels.h"
 
@@ -635,11 +633,21 @@ static hipError_t lg_inst(LgArgs a, hipStream_t st) {
   return hipGetLastError();
 }
 
+constexpr uint32_t kLgRound = 512;  // blocks resident at once: two on each CU
+
 template <int BITS, int G, bool GU>
 static hipError_t lg_shape(const LgArgs& a, hipStream_t st) {
-  // K split over the block's waves from 1024 inputs on (at least two steps
-  // per wave); below, the waves split the columns.
-  if (a.K >= 1024) return lg_inst<BITS, G, GU, 4, 8>(a, st);
+  // Narrow waves (2, then 4 tiles) while their blocks fit the chip at once:
+  // a small call is the latency of its steps, and a step of 8 tiles takes
+  // 2.5 us (16 rows, 2048 -> 4096: 10.8 us with 2 tiles, 13.1 with 4, 17.8
+  // with 8; 128 rows 20.9, 18.4, 20.1; 256 rows 32.5, 27.0, 26.2). K is
+  // split over the block's waves as well, but for calls of more blocks with
+  // less than two steps per wave, whose waves split the columns (2560 x 640
+  // down, 512 tokens: 178 us against 270).
+  auto blocks = [&](uint32_t nt) { return a.n_items * ((a.cols * (GU ? 2 : 1) + nt * 16 - 1) / (nt * 16)); };
+  if (blocks(2) <= kLgRound) return lg_inst<BITS, G, GU, 4, 2>(a, st);
+  if (blocks(4) <= kLgRound) return lg_inst<BITS, G, GU, 4, 4>(a, st);
+  if (a.K >= 1024 || blocks(8) <= kLgRound) return lg_inst<BITS, G, GU, 4, 8>(a, st);
   return lg_inst<BITS, G, GU, 1, 8>(a, st);
 }
 
@@ -648,6 +656,46 @@ static hipError_t lg_gemm(const LgArgs& a, uint32_t bits, uint32_t G, hipStream_
   if (bits == 4)
     return G == 32 ? lg_shape<4, 32, GU>(a, st) : G == 64 ? lg_shape<4, 64, GU>(a, st) : lg_shape<4, 128, GU>(a, st);
   return G == 32 ? lg_shape<3, 32, GU>(a, st) : G == 64 ? lg_shape<3, 64, GU>(a, st) : lg_shape<3, 128, GU>(a, st);
+}
+
+// Dense: y[n, out_dim] = x[n, in_dim] . dequant(W)^T.
+uint64_t limb_qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens) {
+  return lg_rows_bytes(n_tokens, in_dim, group, nullptr, nullptr);
+}
+
+// Whether the limb GEMM is the faster one where k_pf_mm has tiles too (at
+// most 8192 inputs). k_pf_mm walks 32-row x 256-column units on one block
+// per CU, each XCD over its own row blocks: a unit's whole K is its latency,
+// and with fewer than 256 rows XCDs stay idle. us, limb against k_pf_mm:
+// 2048 -> 4096 at 16 / 128 / 256 / 512 rows 10.8 / 18.7 / 26.3 / 43.4 against
+// 133 / 48.5 / 28.4 / 30.3; 4096 -> 1024 at 1000 rows 46.9 against 55.4; 512
+// -> 2048 at 256 / 512 rows 10.2 / 13.4 against 11.4 / 12.0; 2048 -> 152064
+// at 128 / 192 rows 334 / 495 against 433 / 432. So: one round of blocks of 8
+// tiles (half a round below 1024 inputs), or up to 128 rows.
+bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t n) {
+  const uint64_t blocks = (uint64_t)((n + kLgM - 1) / kLgM) * ((out_dim + 127) / 128);
+  return in_dim <= 8192 && (n <= 128 || blocks <= (in_dim < 1024 ? kLgRound / 2 : kLgRound));
+}
+
+hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,
+                           uint8_t* ws, hipStream_t st) {
+  LgRows r;
+  lg_rows_bytes(n, in_dim, w.group, ws, &r);
+  const hipError_t e = lg_prep(nullptr, x, false, n, in_dim, w.group, r, st);
+  if (e != hipSuccess) return e;
+  LgArgs a{};
+  a.base = w.codes;
+  a.s[0] = (uint64_t)((const uint8_t*)w.scales - w.codes);
+  a.b[0] = (uint64_t)((const uint8_t*)w.biases - w.codes);
+  a.cols = out_dim;
+  a.K = in_dim;
+  a.limbs = r.limbs;
+  a.xsum = r.xsum;
+  a.xexp = r.xexp;
+  a.n_items = (n + kLgM - 1) / kLgM;
+  a.n_rows = n;
+  a.out = y;
+  return lg_gemm<false>(a, w.bits, w.group, st);
 }
 
 struct LgPrefill {

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import rel_err
+from helpers import gen_quant_matrix, rel_err
+from test_gpu_decode import dev, oracle_matvec, qweights
 from test_gpu_prefill import _case, _torch, host
 
 pytestmark = pytest.mark.gpu
@@ -73,3 +74,34 @@ def test_limb_prefill_workspace_alignment_and_nonfinite_rows(kernels):
     rest = [t for t in range(n) if t not in (4, 9)]
     assert np.all(np.isnan(out[[4, 9]]))
     assert np.array_equal(out[rest], got[rest])
+
+
+@pytest.mark.parametrize("out_dim,in_dim,group,bits,n", [
+    (31, 32, 32, 4, 2),       # fewer columns than a tile, one chunk
+    (33, 96, 32, 3, 16),      # one column past two tiles, a full row tile
+    (640, 2560, 64, 4, 17),   # 2 tiles per wave, one row past a row tile
+    (1000, 704, 64, 3, 50),   # half a step at the end of K
+    (8200, 1152, 128, 4, 33), # 4 tiles per wave, 9 groups
+    (16500, 320, 64, 4, 40),  # 8 tiles, K split, 2.5 steps over four waves
+    (32900, 640, 32, 3, 30),  # more blocks than fit at once: columns split
+    (16640, 8192, 32, 4, 20), # largest scale area
+    (512, 2048, 64, 4, 100),  # a shape with bf16 tiles
+    (4096, 2048, 64, 4, 257), # one row block past the rule: the bf16 tiles
+])
+def test_limb_qmm_matches_oracle(kernels, out_dim, in_dim, group, bits, n):
+    torch = _torch()
+    rng = np.random.default_rng(out_dim + 3 * in_dim + 7 * n + bits)
+    codes, s, b = gen_quant_matrix(rng, out_dim, in_dim, group, bits)
+    x = rng.standard_normal((n, in_dim)).astype(np.float32)
+    x[0, 5] = 1000.0  # an outlier channel: one exponent per row
+    w = qweights(codes, s, b, group, bits)
+    y = torch.full((n, out_dim), 7.0, dtype=torch.float32, device="cuda")
+    ws = torch.empty(kernels.qmm_workspace_size(in_dim, group, n), dtype=torch.uint8, device="cuda")
+    assert kernels.qmm(w, dev(x), y, out_dim, in_dim, n, ws) == 0
+    got = host(y)
+    rows = sorted({0, n // 2, n - 1})
+    worst = max(rel_err(got[t], oracle_matvec(codes, s, b, in_dim, out_dim, group, bits, x[t])[0]) for t in rows)
+    print(f"limb qmm {n}x{in_dim} -> {out_dim} g{group} {bits}-bit: worst rel_err {worst:.3e}")
+    assert np.all(np.isfinite(got))
+    # The bf16 tiles split x into bf16 pairs: 2^-17 per value.
+    assert worst <= (1e-4 if n == 257 else TOL)
