@@ -264,12 +264,12 @@ __global__ __launch_bounds__(256) void k_lg_prep(LgRoute rt, uint32_t nb_route, 
 // What bounds it: the fold of the limb sums (24 VALU instructions per tile
 // and group of 64, 33 with the unpacking, against 4 MFMAs) and, with two
 // waves per SIMD, what a unit spends before its first step. 512 tokens,
-// 2560 x 640, 512 experts, top-10 (654 items of 16 rows): gate/up 350 us,
-// down 178 us; the VALU is busy half of that, HBM reads run at 2.5 TB/s.
+// 2560 x 640, 512 experts, top-10 (654 items of 16 rows): gate/up 335 us,
+// down 172 us; the VALU is busy half of that, HBM reads run at 2.5 TB/s.
 // Steps, gate/up us: operand-order loads (64 cache accesses per load instead
 // of 16) 455; memory-order loads and a lane permute 367; the next group's
 // MFMAs ahead of a fold, one set of weight registers re-filled tile by tile
-// 359; bias first and two sums per output 350.
+// 359; bias first and two sums per output 350; the scales' loads together 335.
 // ---------------------------------------------------------------------------
 struct LgArgs {
   const uint8_t* base;  // expert e at base + e * stride
@@ -353,16 +353,38 @@ __global__ __launch_bounds__(256, 2) void k_lg(LgArgs a) {
 
   // Scales then biases of the block's rows, per matrix: LDS [m][s, b][row][gpr].
   const uint32_t seg = lg_scale_lds(COLB, gpr), bytes = rowsb * gpr * 2;
+  const uint8_t* sb[2 * NM];
+  uintptr_t al = 0;
 #pragma unroll
   for (int m = 0; m < 2 * NM; ++m) {
-    const uint8_t* const src = blob + (m & 1 ? a.b[m / 2] : a.s[m / 2]) + (uint64_t)colb * gpr * 2;
-    uint8_t* const dst = lds + m * seg;
-    const bool al = ((uintptr_t)src & 15) == 0;
-    const uint32_t whole = al ? bytes / 16 * 16 : 0u;
-    for (uint32_t i = tid * 16; i < whole; i += 4096) *reinterpret_cast<u32x4*>(dst + i) = *reinterpret_cast<const u32x4*>(src + i);
-    for (uint32_t i = whole + tid * 2; i < bytes; i += 512)
-      *reinterpret_cast<uint16_t*>(dst + i) = *reinterpret_cast<const uint16_t*>(src + i);
+    sb[m] = blob + (m & 1 ? a.b[m / 2] : a.s[m / 2]) + (uint64_t)colb * gpr * 2;
+    al |= (uintptr_t)sb[m];
   }
+  // 16-byte pieces of all of them as one list, SU loads per thread in flight
+  // (one at a time, each waited for by its LDS write, took 5.4 us of a
+  // unit's 22 at 2560 x 640); then what is left of each by two bytes.
+  const uint32_t whole = al % 16 == 0 ? bytes / 16 : 0u;
+  constexpr uint32_t SU = NT >= 8 ? 6 : 2;
+  for (uint32_t p0 = tid; p0 < whole * 2 * NM; p0 += 256 * SU) {
+    u32x4 v[SU];
+    uint32_t dst[SU];
+#pragma unroll
+    for (uint32_t j = 0; j < SU; ++j) {
+      uint32_t i = min(p0 + 256 * j, whole * 2 * NM - 1), m = 0;
+      const uint8_t* src = sb[0];
+#pragma unroll
+      for (int k = 1; k < 2 * NM; ++k)
+        if (i >= whole) i -= whole, m = k, src = sb[k];
+      v[j] = *reinterpret_cast<const u32x4*>(src + i * 16);
+      dst[j] = m * seg + i * 16;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < SU; ++j) *reinterpret_cast<u32x4*>(lds + dst[j]) = v[j];
+  }
+#pragma unroll
+  for (int m = 0; m < 2 * NM; ++m)
+    for (uint32_t i = whole * 16 + tid * 2; i < bytes; i += 512)
+      *reinterpret_cast<uint16_t*>(lds + m * seg + i) = *reinterpret_cast<const uint16_t*>(sb[m] + i);
 
   // Group sums of the bias term, four of this wave's groups per MFMA: lane
   // block kb of batch q takes the (4 q + kb)-th; zero past the last.
