@@ -390,8 +390,10 @@ int smoe_router(smoe_handle* h, const float* router_w, const float* x, uint32_t 
     logits = h->logits;
   }
   if (int rc = use_device(h)) return rc;
-  hipError_t e = launch_router_logits(router_w, nullptr, x, n_tokens, n_experts, hidden, logits,
-                                      nullptr, h->stream);
+  hipError_t e = router_mm_supported(n_tokens, n_experts, hidden)
+                     ? launch_router_mm(router_w, x, n_tokens, n_experts, hidden, logits, h->stream)
+                     : launch_router_logits(router_w, nullptr, x, n_tokens, n_experts, hidden, logits, nullptr,
+                                            h->stream);
   if (e != hipSuccess) return SMOE_ERR_HIP;
   RouteOut ro{};
   ro.idx = idx;

@@ -245,6 +245,10 @@ hipError_t launch_router_logits(const float* W, const float* gate_w, const float
                                 float* logits, float* gate_scores, hipStream_t st,
                                 const uint16_t* norm_w = nullptr, float eps = 0.f, float* x_out = nullptr,
                                 const Q8Rows& Wq = Q8Rows{}, const Q8Rows& gq = Q8Rows{});
+// The same for many tokens (f32 router, no gate, no norm) on MFMA (router.hip).
+bool router_mm_supported(uint32_t n_tokens, uint32_t n_experts, uint32_t hidden);
+hipError_t launch_router_mm(const float* W, const float* x, uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
+                            float* logits, hipStream_t st);
 // Softmax (optional) + running-min top-k + optional renorm, one wave per token.
 hipError_t launch_topk(const float* scores, uint32_t n_tokens, uint32_t n, uint32_t k,
                        bool softmax, bool normalize, const RouteOut& out, hipStream_t st);

@@ -205,4 +205,155 @@ hipError_t launch_noaux_topk(const float* logits, const float* bias, uint32_t n_
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// Router logits of many tokens: logits[t, e] = W[e] . x[t] in f32 on
+// v_mfma_f32_16x16x4_f32. A block of eight waves holds 16 tokens x 32 experts;
+// the waves split the inputs, 32 at a time, each copying its own piece of
+// the 16 x rows and 32 router rows to LDS (LDS DMA in memory order, four lanes
+// per row's 64 bytes) one piece ahead and reading it back in operand order,
+// so the loop has no block barrier. 16-byte part p of row r is stored at part
+// p ^ (r / 4 % 4): the 16 rows of an operand read fall on all banks.
+//
+// Rounding: an accumulator runs over 8 inputs (two MFMAs) and the sums are
+// then added pairwise (a binary tree over a wave's inputs, then over the
+// waves), as the one-row kernel's lanes are, not along one chain of `hidden`
+// additions.
+//
+// 512 tokens, 256 experts, hidden 2048: 94 us with a block per (token, expert
+// row), each reading both rows again (2 GB through L2); 12.4 us
+// here, the limit of its chain of eight pieces per wave (the matrix cores are
+// busy 3.5 us of it).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kRlT = 16, kRlE = 32, kRlW = 8;           // tokens, experts, waves per block
+constexpr uint32_t kRlK = 32;                                // inputs per piece
+constexpr uint32_t kRlRows = kRlT + kRlE;                    // rows of a piece
+constexpr uint32_t kRlPiece = kRlRows * kRlK * 4;            // bytes
+constexpr uint32_t kRlRing = 2;                              // pieces in LDS per wave
+constexpr uint32_t kRlLds = kRlW * kRlRing * kRlPiece;
+static_assert(kRlLds <= 160 * 1024, "LDS per CU");
+static_assert(kRlLds >= kRlW * 2 * 64 * 16, "the waves' sums fit over the pieces");
+
+__global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict__ W, const float* __restrict__ x,
+                                                         uint32_t n, uint32_t E, uint32_t H,
+                                                         float* __restrict__ logits) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t c16 = lane & 15, kb = lane >> 4;
+  const uint32_t ne = (E + kRlE - 1) / kRlE;
+  const uint32_t t0 = blockIdx.x / ne * kRlT, e0 = blockIdx.x % ne * kRlE;
+  uint8_t* const mine = lds + wave * kRlRing * kRlPiece;
+  // Lane l copies part l % 4 of row l / 4 of each group of 16 rows; rows past
+  // the end repeat the last (their sums are dropped).
+  const uint32_t lr = lane >> 2, part = ((lane & 3) ^ (lr >> 2)) * 16;
+  const uint8_t* src[3];
+  src[0] = reinterpret_cast<const uint8_t*>(x + (size_t)min(t0 + lr, n - 1) * H) + part;
+  src[1] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + lr, E - 1) * H) + part;
+  src[2] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + 16 + lr, E - 1) * H) + part;
+  // Piece i of this wave: inputs [32 (wave + 8 i), + 32), as two 16-input
+  // columns of 64 bytes per row.
+  constexpr uint32_t NC = kRlK / 16;
+  const uint32_t np = (H / kRlK + kRlW - 1 - wave) / kRlW;
+  auto copy = [&](uint32_t i) {
+    const uint32_t k0 = (wave + kRlW * i) * (kRlK * 4);
+    uint8_t* const dst = mine + i % kRlRing * kRlPiece;
+#pragma unroll
+    for (uint32_t g = 0; g < 3; ++g)
+#pragma unroll
+      for (uint32_t c = 0; c < NC; ++c) dma16(src[g] + k0 + c * 64, dst + (g * NC + c) * 1024);
+  };
+  f32x4 sum[2][8];  // pairwise tree of each tile: level v holds 2^v pieces' sums
+  uint32_t have = 0;
+  if (np) copy(0);
+  const uint32_t rd = c16 * 64 + ((kb ^ (c16 >> 2)) * 16);  // operand part of lane (row, kb)
+  for (uint32_t i = 0; i < np; ++i) {
+    // The reads of the piece before are done, its buffer takes the next
+    // piece's copies; then this piece has landed when this wave's copies of
+    // it have (the next piece's six stay in flight; a third buffer 13.0 us).
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + 1 < np) {
+      copy(i + 1);
+      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const uint8_t* const p = mine + i % kRlRing * kRlPiece + rd;
+    static_assert(3 * NC == 6, "copies per piece");
+    f32x4 leaf[2][2 * NC];
+#pragma unroll
+    for (uint32_t c = 0; c < NC; ++c) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(p + c * 1024);
+#pragma unroll
+      for (uint32_t t = 0; t < 2; ++t) {
+        const f32x4 b = *reinterpret_cast<const f32x4*>(p + ((t + 1) * NC + c) * 1024);
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        leaf[t][2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, z, 0, 0, 0);
+        leaf[t][2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, z, 0, 0, 0);
+        leaf[t][2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, leaf[t][2 * c], 0, 0, 0);
+        leaf[t][2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, leaf[t][2 * c + 1], 0, 0, 0);
+      }
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (uint32_t t = 0; t < 2; ++t) s[t] = (leaf[t][0] + leaf[t][1]) + (leaf[t][2] + leaf[t][3]);
+    // Binary counter: carry the sum up past the levels that are full.
+    bool done = false;
+#pragma unroll
+    for (uint32_t v = 0; v < 8; ++v) {
+      if (done) continue;
+      if (have >> v & 1) {
+        s[0] += sum[0][v];
+        s[1] += sum[1][v];
+      } else {
+        sum[0][v] = s[0];
+        sum[1][v] = s[1];
+        done = true;
+      }
+    }
+    ++have;
+  }
+  f32x4 tot[2] = {};
+#pragma unroll
+  for (uint32_t v = 0; v < 8; ++v)
+    if (have >> v & 1) {
+      tot[0] += sum[0][v];
+      tot[1] += sum[1][v];
+    }
+  // The waves' sums, pairwise.
+  __syncthreads();
+  f32x4* const red = reinterpret_cast<f32x4*>(lds);
+  red[(wave * 2 + 0) * 64 + lane] = tot[0];
+  red[(wave * 2 + 1) * 64 + lane] = tot[1];
+  __syncthreads();
+  if (wave < 2) {
+    const f32x4* const p = red + wave * 64 + lane;
+    const f32x4 v = ((p[0] + p[128]) + (p[256] + p[384])) + ((p[512] + p[640]) + (p[768] + p[896]));
+    const uint32_t e = e0 + wave * 16 + c16;
+    if (e < E)
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t t = t0 + kb * 4 + i;
+        if (t < n) logits[(size_t)t * E + e] = v[i];
+      }
+  }
+}
+
+// Whether a call runs on k_router_mm: whole pieces, no more of them per wave
+// than the tree has room for, and enough logits: a wave's chain of pieces costs
+// 7 us more than one row's block at hidden 2048 (23 at 7168), the one-row
+// kernel 0.27 us per million products, so the line is at about 2^14 logits
+// whatever the hidden size.
+bool router_mm_supported(uint32_t n_tokens, uint32_t n_experts, uint32_t hidden) {
+  return (uint64_t)n_tokens * n_experts >= (1u << 14) && hidden % kRlK == 0 && hidden <= 32768;
+}
+
+hipError_t launch_router_mm(const float* W, const float* x, uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
+                            float* logits, hipStream_t st) {
+  static std::atomic<uint64_t> raised{0};
+  const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_router_mm), kRlLds, raised);
+  if (e != hipSuccess) return e;
+  const uint32_t blocks = (n_tokens + kRlT - 1) / kRlT * ((n_experts + kRlE - 1) / kRlE);
+  hipLaunchKernelGGL(k_router_mm, dim3(blocks), dim3(64 * kRlW), kRlLds, st, W, x, n_tokens, n_experts, hidden, logits);
+  return hipGetLastError();
+}
+
 }  // namespace smoe

@@ -1,0 +1,39 @@
+"""smoe_router over many tokens (k_router_mm) at the edges of its tiles: the
+logits against float64, the routing against smoe_softmax_topk of the returned
+logits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,E,H", [
+    (129, 127, 96),     # one logit short of the rule: a block per row
+    (129, 128, 96),     # three pieces over eight waves, one token past a tile
+    (33, 500, 32),      # one piece, experts not a multiple of a tile
+    (17, 1000, 2560),   # one token past a tile
+    (1024, 16, 2080),   # half an expert tile, 65 pieces
+    (500, 256, 2048),
+    (70, 256, 100),     # not whole pieces: a block per row
+])
+def test_router_many_tokens(kernels, n, E, H):
+    import torch
+
+    rng = np.random.default_rng(n + E + H)
+    W = (rng.standard_normal((E, H)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((n, H)).astype(np.float32)
+    x[n // 2, 3] = 1e4
+    k = min(8, E)
+    wd, xd = torch.from_numpy(W).cuda(), torch.from_numpy(x).cuda()
+    new = lambda dt, *s: torch.zeros(s, dtype=dt, device="cuda")
+    idx, w, lg = new(torch.int32, n, k), new(torch.float32, n, k), new(torch.float32, n, E)
+    assert kernels.router(wd, xd, n, E, H, k, True, idx, w, lg) == 0
+    idx2, w2 = new(torch.int32, n, k), new(torch.float32, n, k)
+    assert kernels.softmax_topk(lg, n, E, k, True, idx2, w2) == 0
+    kernels.sync()
+    assert torch.equal(idx, idx2) and torch.equal(w, w2)
+    want = x.astype(np.float64) @ W.astype(np.float64).T
+    # Rounding of chains of 8 products and log2(H / 8) <= 13 pairwise levels,
+    # 2^-24 of the partial sums each, which sum |w x| bounds.
+    bound = 21 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T)
+    assert np.all(np.abs(lg.cpu().numpy() - want) <= bound)
