@@ -486,13 +486,9 @@ int smoe_experts_decode(smoe_handle* h, const smoe_expert_shape* shape,
   tab.shared_gate = shared_gate_score;
   if (int rc = use_device(h)) return rc;
   const BlobGeom g = blob_geom(shape->hidden, shape->inter, shape->group, shape->bits);
-  bool uns = false;
-  hipError_t e = launch_gateup(g, g, nullptr, tab, k, input, h->act, h->stream, &uns);
-  if (uns) return SMOE_ERR_UNSUPPORTED_SHAPE;
+  hipError_t e = launch_gateup(g, g, nullptr, tab, k, input, h->act, h->stream);
   if (e != hipSuccess) return SMOE_ERR_HIP;
-  e = launch_down_combine(g, g, nullptr, tab, k, h->act, h_mid, shared_out, hidden_out, h->stream,
-                          &uns);
-  if (uns) return SMOE_ERR_UNSUPPORTED_SHAPE;
+  e = launch_down_combine(g, g, nullptr, tab, k, h->act, h_mid, shared_out, hidden_out, h->stream);
   return hip_status(e);
 }
 
@@ -575,13 +571,9 @@ static int decode_layer(smoe_handle* h, const smoe_layer* L, const float* input,
   FfnTable tv{};
   tv.k = L->k;
   const uint32_t n_slots = L->k + (L->shared_expert ? 1 : 0);
-  bool uns = false;
-  e = launch_gateup(g, gs, h->table, tv, n_slots, input, h->act, h->stream, &uns);
-  if (uns) return SMOE_ERR_UNSUPPORTED_SHAPE;
+  e = launch_gateup(g, gs, h->table, tv, n_slots, input, h->act, h->stream);
   if (e != hipSuccess) return SMOE_ERR_HIP;
-  e = launch_down_combine(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out,
-                          h->stream, &uns);
-  if (uns) return SMOE_ERR_UNSUPPORTED_SHAPE;
+  e = launch_down_combine(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out, h->stream);
   return hip_status(e);
 }
 
@@ -835,9 +827,9 @@ int smoe_moe_prefill(smoe_handle* h, const smoe_expert_shape* shape, const void*
     return SMOE_ERR_MISALIGNED;
   if (!prefill_supported(shape->hidden, shape->inter, shape->group, shape->bits, n_tokens, n_experts, k)) {
     // Shapes without bf16 / fp16 grouped-GEMM tiles: grouped on the int8
-    // matrix cores from three tokens on; fewer (2560 x 640, top-10: one 33 us
-    // against 48, two 65 against 49, three 96 against 57; 2048 x 512, top-8:
-    // two 35 against 41, eight 134 against 51), or a workspace too small for
+    // matrix cores from three tokens on; fewer (2560 x 640, top-10: one 21 us
+    // against 46, two 41 against 48, three 61 against 53; 2048 x 512, top-8:
+    // two 27 against 41, three 41 against 34), or a workspace too small for
     // the grouped call, one token at a time through the per-phase decode
     // kernels.
     if (n_tokens > 2 &&
@@ -851,13 +843,9 @@ int smoe_moe_prefill(smoe_handle* h, const smoe_expert_shape* shape, const void*
     if (workspace_bytes < prefill_tokens_workspace(shape->hidden, shape->inter, n_tokens, k, x_is_bf16 != 0))
       return SMOE_ERR_WORKSPACE_TOO_SMALL;
     if (int rc = use_device(h)) return rc;
-    bool unsupported = false;
-    const hipError_t e = launch_prefill_tokens(
+    return hip_status(launch_prefill_tokens(
         blob_geom(shape->hidden, shape->inter, shape->group, shape->bits), (const uint8_t*)experts, stride,
-        n_experts, idx, weights, x, x_is_bf16 != 0, n_tokens, k, out_sum, (uint8_t*)workspace, h->err, h->stream,
-        &unsupported);
-    if (unsupported) return SMOE_ERR_UNSUPPORTED_SHAPE;
-    return hip_status(e);
+        n_experts, idx, weights, x, x_is_bf16 != 0, n_tokens, k, out_sum, (uint8_t*)workspace, h->err, h->stream));
   }
   PfArgs a{};
   const uint64_t need = prefill_workspace(shape->hidden, shape->inter, shape->group, n_tokens,

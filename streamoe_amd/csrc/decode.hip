@@ -7,11 +7,10 @@
 //   k_topk           softmax + running-minimum top-k + renorm, one wave
 //                    per token, exact slot order of the reference.
 //   k_gateup         fused gate + up + SwiGLU over all routed slots and
-//                    the shared expert; one wave reads whole rows with
-//                    one 16-byte (4-bit) / 12-byte (3-bit) load per lane.
-//   k_down_combine   down projection of every slot for a few output rows
-//                    plus the fixed-order weighted combine and residual,
-//                    no atomics.
+//                    the shared expert at hidden 4096 (phase.hip otherwise).
+//   k_down_combine   down projection of every slot for one output row plus
+//                    the fixed-order weighted combine and residual, where
+//                    phase.hip's block would not fit.
 #include "common.h"
 #include "kernels.h"
 #include "topk.h"
@@ -731,36 +730,36 @@ hipError_t launch_topk(const float* scores, uint32_t n_tokens, uint32_t n, uint3
 }
 
 // ---------------------------------------------------------------------------
-// Fused gate/up + SwiGLU.  CPR = hidden / 32. One block = one wave handling
-// RW rows (gate and up) of one slot; the block index enumerates
-// (slot, row tile), slots 0..k-1 routed, slot k the shared expert.
+// Fused gate/up + SwiGLU at hidden 4096: one wave per 2 rows (gate and up) of
+// one slot, a whole wave per row, two chunks per lane; the block index
+// enumerates (slot, row pair), slots 0..k-1 routed, slot k the shared
+// expert. Every other width, and every call's down rows, run in phase.hip: at
+// this one, whole waves per row and x in registers are the faster (gate/up
+// and down, 512 experts, top-10, inter 1024: 31 us against 34 with 16 lanes
+// per row).
 // ---------------------------------------------------------------------------
-template <int BITS, int CPR, int P, bool PAD>
-__device__ __forceinline__ void gateup_body(const uint8_t* __restrict__ blob, const BlobGeom& g,
-                                            uint32_t row0, const float (&xr)[CPR < 64 ? 1 : CPR / 64][kChunk],
-                                            const float (&xs)[CPR < 64 ? 1 : CPR / 64],
+constexpr int kGuChunks = 128, kGuCPL = kGuChunks / kWave, kGuRows = 2;
+
+template <int BITS>
+__device__ __forceinline__ void gateup_body(const uint8_t* __restrict__ blob, const BlobGeom& g, uint32_t row0,
+                                            const float (&xr)[kGuCPL][kChunk], const float (&xs)[kGuCPL],
                                             float* __restrict__ act_slot) {
-  constexpr int L = CPR < kWave ? CPR : kWave;
-  constexpr int CPL = CPR / L;
-  constexpr int RPP = kWave / L;
   constexpr int CB = chunk_bytes<BITS>();
-  const uint32_t cpr = PAD ? g.hidden / kChunk : (uint32_t)CPR;
-  const uint32_t ROW_BYTES = cpr * CB;
+  constexpr uint32_t ROW_BYTES = kGuChunks * CB;
   const int lane = threadIdx.x & 63;
-  const int lrow = lane / L, lch = lane % L;
   const uint32_t gpr = g.hidden / g.group;
   const uint32_t cpg_shift = __builtin_ctz(g.group / kChunk);
   const uint32_t inter = g.inter;
 
-  Raw<BITS> rg[P][CPL], ru[P][CPL];
-  float sg[P][CPL], bg[P][CPL], su[P][CPL], bu[P][CPL];
+  Raw<BITS> rg[kGuRows][kGuCPL], ru[kGuRows][kGuCPL];
+  float sg[kGuRows][kGuCPL], bg[kGuRows][kGuCPL], su[kGuRows][kGuCPL], bu[kGuRows][kGuCPL];
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    uint32_t row = row0 + p * RPP + lrow;
+  for (int p = 0; p < kGuRows; ++p) {
+    uint32_t row = row0 + p;
     row = row < inter ? row : inter - 1;
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      const uint32_t c = PAD ? pad_chunk(lch + L * i, cpr) : lch + L * i;
+    for (int i = 0; i < kGuCPL; ++i) {
+      const uint32_t c = lane + kWave * i;
       const size_t off = (size_t)row * ROW_BYTES + c * CB;
       rg[p][i] = load_raw<BITS>(blob + g.w[0] + off);
       ru[p][i] = load_raw<BITS>(blob + g.w[1] + off);
@@ -771,136 +770,66 @@ __device__ __forceinline__ void gateup_body(const uint8_t* __restrict__ blob, co
       bu[p][i] = bf16f(*reinterpret_cast<const uint16_t*>(blob + g.b[1] + gi));
     }
   }
-  if constexpr (L == kWave && P == 4) {
-    // Whole-wave rows: the four gate and four up rows are reduced together
-    // (after the permlane swaps the 16-lane rows hold rows 0, 2, 1, 3), and
-    // one SwiGLU per lane serves the four outputs.
-    float pg[P], pu[P];
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      pg[p] = 0.f;
-      pu[p] = 0.f;
+  for (int p = 0; p < kGuRows; ++p) {
+    float pg = 0.f, pu = 0.f;
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) {
-        pg[p] += chunk_dot<BITS>(rg[p][i], xr[i], xs[i], sg[p][i], bg[p][i]);
-        pu[p] += chunk_dot<BITS>(ru[p][i], xr[i], xs[i], su[p][i], bu[p][i]);
-      }
+    for (int i = 0; i < kGuCPL; ++i) {
+      pg += chunk_dot<BITS>(rg[p][i], xr[i], xs[i], sg[p][i], bg[p][i]);
+      pu += chunk_dot<BITS>(ru[p][i], xr[i], xs[i], su[p][i], bu[p][i]);
     }
-    const float gsum = row_sum16_all(swap16_add(swap32_add(pg[0], pg[1]), swap32_add(pg[2], pg[3])));
-    const float usum = row_sum16_all(swap16_add(swap32_add(pu[0], pu[1]), swap32_add(pu[2], pu[3])));
-    const int r16 = lane >> 4;
-    const uint32_t row = row0 + ((r16 >> 1) | ((r16 & 1) << 1));
-    if ((lane & 15) == 0 && row < inter) act_slot[row] = silu_mul(gsum, usum);
-  } else {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      float pg = 0.f, pu = 0.f;
-#pragma unroll
-      for (int i = 0; i < CPL; ++i) {
-        pg += chunk_dot<BITS>(rg[p][i], xr[i], xs[i], sg[p][i], bg[p][i]);
-        pu += chunk_dot<BITS>(ru[p][i], xr[i], xs[i], su[p][i], bu[p][i]);
-      }
-      const float gsum = group_sum<L>(pg);
-      const float usum = group_sum<L>(pu);
-      const uint32_t row = row0 + p * RPP + lrow;
-      if (lch == 0 && row < inter) act_slot[row] = silu_mul(gsum, usum);
-    }
+    const float gsum = group_sum<kWave>(pg);
+    const float usum = group_sum<kWave>(pu);
+    if (lane == 0 && row0 + p < inter) act_slot[row0 + p] = silu_mul(gsum, usum);
   }
 }
 
-template <int BITS, int CPR, int P, bool PAD>
-__global__ __launch_bounds__(64) void k_gateup(BlobGeom routed, BlobGeom shared,
-                                               const FfnTable* __restrict__ tab_dev,
-                                               FfnTable tab_val, uint32_t tiles_per_slot,
-                                               const float* __restrict__ x,
+template <int BITS>
+__global__ __launch_bounds__(64) void k_gateup(BlobGeom routed, BlobGeom shared, const FfnTable* __restrict__ tab_dev,
+                                               FfnTable tab_val, uint32_t tiles_per_slot, const float* __restrict__ x,
                                                float* __restrict__ act) {
-  constexpr int L = CPR < kWave ? CPR : kWave;
-  constexpr int CPL = CPR / L;
-  constexpr int RPP = kWave / L;
-  constexpr uint32_t RW = RPP * P;  // rows per wave
   const int lane = threadIdx.x & 63;
-  const int lch = lane % L;
   const uint32_t slot = blockIdx.x / tiles_per_slot;
   const uint32_t tile = blockIdx.x % tiles_per_slot;
   const uint32_t k = tab_dev ? tab_dev->k : tab_val.k;
   const uint8_t* blob = tab_dev ? tab_dev->blob[slot] : tab_val.blob[slot];
 
-  float xr[CPL][kChunk];
-  float xs[CPL];
+  float xr[kGuCPL][kChunk];
+  float xs[kGuCPL];
 #pragma unroll
-  for (int i = 0; i < CPL; ++i) {
-    if (PAD)
-      load_x32_pad(x, lch + L * i, routed.hidden / kChunk, xr[i]);
-    else
-      load_x32(x + (size_t)(lch + L * i) * kChunk, xr[i]);
+  for (int i = 0; i < kGuCPL; ++i) {
+    load_x32(x + (size_t)(lane + kWave * i) * kChunk, xr[i]);
     xs[i] = xsum(xr[i]);
   }
-  const uint32_t row0 = tile * RW;
-  if (slot < k) {
-    if (row0 >= routed.inter) return;
-    gateup_body<BITS, CPR, P, PAD>(blob, routed, row0, xr, xs, act + (size_t)slot * routed.inter);
-  } else {
-    if (row0 >= shared.inter) return;
-    gateup_body<4, CPR, P, PAD>(blob, shared, row0, xr, xs, act + (size_t)slot * routed.inter);
-  }
-}
-
-template <int BITS, int CPR, bool PAD = false>
-static hipError_t gateup_inst(const BlobGeom& routed, const BlobGeom& shared,
-                              const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t n_slots,
-                              const float* x, float* act, hipStream_t st) {
-  constexpr int L = CPR < kWave ? CPR : kWave;
-  constexpr int RPP = kWave / L;
-  constexpr int P = CPR / L >= 4 ? 2 : 4;  // rows per lane group: 4, or 2 with 4 chunks per lane
-  const uint32_t rw = RPP * P;
-  const uint32_t tiles = (routed.inter + rw - 1) / rw;
-  hipLaunchKernelGGL((k_gateup<BITS, CPR, P, PAD>), dim3(tiles * n_slots), dim3(64), 0, st, routed,
-                     shared, tab_dev, tab_val, tiles, x, act);
-  return hipGetLastError();
-}
-
-template <int BITS>
-static hipError_t gateup_bits(const BlobGeom& routed, const BlobGeom& shared,
-                              const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t n_slots,
-                              const float* x, float* act, hipStream_t st, bool* unsupported) {
-  const uint32_t cpr = routed.hidden / kChunk;
-  switch (cpr) {
-    case 32: return gateup_inst<BITS, 32>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-    case 64: return gateup_inst<BITS, 64>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-    case 128: return gateup_inst<BITS, 128>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-    default: break;
-  }
-  // Other hidden sizes (multiples of 32 up to 8192): the padded instances.
-  if (cpr == 0) {
-    *unsupported = true;
-    return hipSuccess;
-  }
-  if (cpr <= 8) return gateup_inst<BITS, 8, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if (cpr <= 16) return gateup_inst<BITS, 16, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if (cpr <= 32) return gateup_inst<BITS, 32, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if (cpr <= 64) return gateup_inst<BITS, 64, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if (cpr <= 128) return gateup_inst<BITS, 128, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if (cpr <= 256) return gateup_inst<BITS, 256, true>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  *unsupported = true;
-  return hipSuccess;
+  const uint32_t row0 = tile * kGuRows;
+  float* const out = act + (size_t)slot * routed.inter;
+  if (slot < k)
+    gateup_body<BITS>(blob, routed, row0, xr, xs, out);
+  else
+    gateup_body<4>(blob, shared, row0, xr, xs, out);
 }
 
 hipError_t launch_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
-                         const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act,
-                         hipStream_t st, bool* unsupported) {
-  *unsupported = false;
-  return routed.bits == 4
-             ? gateup_bits<4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st, unsupported)
-             : gateup_bits<3>(routed, shared, tab_dev, tab_val, n_slots, x, act, st, unsupported);
+                         const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  if (routed.hidden != kGuChunks * kChunk) return launch_ph_gateup(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+  const uint32_t tiles = (routed.inter + kGuRows - 1) / kGuRows;
+  if (routed.bits == 4)
+    hipLaunchKernelGGL(k_gateup<4>, dim3(tiles * n_slots), dim3(64), 0, st, routed, shared, tab_dev, tab_val, tiles, x, act);
+  else
+    hipLaunchKernelGGL(k_gateup<3>, dim3(tiles * n_slots), dim3(64), 0, st, routed, shared, tab_dev, tab_val, tiles, x, act);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// Down + combine.  CPR = inter / 32. One wave = RPP output rows; it loads
+// Down + combine where (slots, chunks) exceed a block's LDS in phase.hip
+// (inter > 1920 with 15 or 16 slots). One wave = one output row; it loads
 // every slot's chunk of those rows up front, then reduces slot by slot in
 // the reference's order: moe = fma(out_k, w_k, moe) (deferred.rs:458-466),
 // then the shared term and the residual.
 // ---------------------------------------------------------------------------
-template <int BITS, int CPR, int MAXS, bool PAD>
+constexpr int kDcMaxS = kMaxK;  // routed slots held at once
+
+template <int BITS>
 __global__ __launch_bounds__(64) void k_down_combine(BlobGeom routed, BlobGeom shared,
                                                      const FfnTable* __restrict__ tab_dev,
                                                      FfnTable tab_val,
@@ -908,22 +837,17 @@ __global__ __launch_bounds__(64) void k_down_combine(BlobGeom routed, BlobGeom s
                                                      const float* __restrict__ h_mid,
                                                      const float* __restrict__ shared_out,
                                                      float* __restrict__ hidden_out) {
-  constexpr int L = CPR < kWave ? CPR : kWave;
-  constexpr int CPL = CPR / L;
-  constexpr int RPP = kWave / L;
+  constexpr int MAXS = kDcMaxS;
   constexpr int CB = chunk_bytes<BITS>();
   constexpr int CB4 = chunk_bytes<4>();
-  const uint32_t cpr = PAD ? routed.inter / kChunk : (uint32_t)CPR;
+  const uint32_t cpr = routed.inter / kChunk;  // at most one chunk per lane
   const uint32_t ROW_BYTES = cpr * CB;
   const uint32_t ROW_BYTES4 = cpr * CB4;
   const int lane = threadIdx.x & 63;
-  const int lrow = lane / L, lch = lane % L;
-  const uint32_t H = routed.hidden, I = routed.inter;
+  const uint32_t I = routed.inter;
   const uint32_t gpr = I / routed.group;
   const uint32_t cpg_shift = __builtin_ctz(routed.group / kChunk);
-  uint32_t row = blockIdx.x * RPP + lrow;
-  const bool valid = row < H;
-  row = valid ? row : H - 1;
+  const uint32_t row = blockIdx.x, c = pad_chunk(lane, cpr);
 
   const uint32_t k = tab_dev ? tab_dev->k : tab_val.k;
   const uint32_t has_shared = tab_dev ? tab_dev->has_shared : tab_val.has_shared;
@@ -931,52 +855,36 @@ __global__ __launch_bounds__(64) void k_down_combine(BlobGeom routed, BlobGeom s
   // Every slot up to MAXS is loaded and computed without a branch (slots
   // past k re-read slot k - 1 and are not added), so the loads and lane
   // reductions of different slots overlap instead of running one by one.
-  Raw<BITS> raw[MAXS][CPL];
-  Raw<4> rsh[CPL];
-  float sv[MAXS][CPL], bv[MAXS][CPL], ssh[CPL], bsh[CPL];
+  Raw<BITS> raw[MAXS];
+  Raw<4> rsh;
+  float sv[MAXS], bv[MAXS], ssh = 0.f, bsh = 0.f;
 #pragma unroll
   for (int s = 0; s < MAXS; ++s) {
     const uint32_t sl = (uint32_t)s < k ? (uint32_t)s : k - 1;
     const uint8_t* blob = tab_dev ? tab_dev->blob[sl] : tab_val.blob[sl];
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      const uint32_t c = PAD ? pad_chunk(lch + L * i, cpr) : lch + L * i;
-      raw[s][i] = load_raw<BITS>(blob + routed.w[2] + (size_t)row * ROW_BYTES + c * CB);
-      const size_t gi = ((size_t)row * gpr + (c >> cpg_shift)) * 2;
-      sv[s][i] = bf16f(*reinterpret_cast<const uint16_t*>(blob + routed.s[2] + gi));
-      bv[s][i] = bf16f(*reinterpret_cast<const uint16_t*>(blob + routed.b[2] + gi));
-    }
+    raw[s] = load_raw<BITS>(blob + routed.w[2] + (size_t)row * ROW_BYTES + c * CB);
+    const size_t gi = ((size_t)row * gpr + (c >> cpg_shift)) * 2;
+    sv[s] = bf16f(*reinterpret_cast<const uint16_t*>(blob + routed.s[2] + gi));
+    bv[s] = bf16f(*reinterpret_cast<const uint16_t*>(blob + routed.b[2] + gi));
   }
   if (has_shared) {
     const uint8_t* blob = tab_dev ? tab_dev->blob[k] : tab_val.blob[k];
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      const uint32_t c = PAD ? pad_chunk(lch + L * i, cpr) : lch + L * i;
-      rsh[i] = load_raw<4>(blob + shared.w[2] + (size_t)row * ROW_BYTES4 + c * CB4);
-      const size_t gi = ((size_t)row * gpr + (c >> cpg_shift)) * 2;
-      ssh[i] = bf16f(*reinterpret_cast<const uint16_t*>(blob + shared.s[2] + gi));
-      bsh[i] = bf16f(*reinterpret_cast<const uint16_t*>(blob + shared.b[2] + gi));
-    }
+    rsh = load_raw<4>(blob + shared.w[2] + (size_t)row * ROW_BYTES4 + c * CB4);
+    const size_t gi = ((size_t)row * gpr + (c >> cpg_shift)) * 2;
+    ssh = bf16f(*reinterpret_cast<const uint16_t*>(blob + shared.s[2] + gi));
+    bsh = bf16f(*reinterpret_cast<const uint16_t*>(blob + shared.b[2] + gi));
   }
 
   float o[MAXS];
 #pragma unroll
   for (int s = 0; s < MAXS; ++s) {
     const uint32_t sl = (uint32_t)s < k ? (uint32_t)s : k - 1;
-    float part = 0.f;
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      float a[kChunk];
-      if (PAD)
-        load_x32_pad(act + (size_t)sl * I, lch + L * i, cpr, a);
-      else
-        load_x32(act + (size_t)sl * I + (size_t)(lch + L * i) * kChunk, a);
-      part += chunk_dot<BITS>(raw[s][i], a, xsum(a), sv[s][i], bv[s][i]);
-    }
-    o[s] = part;
+    float a[kChunk];
+    load_x32_pad(act + (size_t)sl * I, lane, cpr, a);
+    o[s] = chunk_dot<BITS>(raw[s], a, xsum(a), sv[s], bv[s]);
   }
 #pragma unroll
-  for (int s = 0; s < MAXS; ++s) o[s] = group_sum<L>(o[s]);
+  for (int s = 0; s < MAXS; ++s) o[s] = group_sum<kWave>(o[s]);
   // moe = fma(out_k, w_k, moe) in slot order (deferred.rs:458-466).
   float moe = 0.f;
 #pragma unroll
@@ -986,17 +894,9 @@ __global__ __launch_bounds__(64) void k_down_combine(BlobGeom routed, BlobGeom s
   }
   float res;
   if (has_shared) {
-    float part = 0.f;
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      float a[kChunk];
-      if (PAD)
-        load_x32_pad(act + (size_t)k * I, lch + L * i, cpr, a);
-      else
-        load_x32(act + (size_t)k * I + (size_t)(lch + L * i) * kChunk, a);
-      part += chunk_dot<4>(rsh[i], a, xsum(a), ssh[i], bsh[i]);
-    }
-    const float sh = group_sum<L>(part);
+    float a[kChunk];
+    load_x32_pad(act + (size_t)k * I, lane, cpr, a);
+    const float sh = group_sum<kWave>(chunk_dot<4>(rsh, a, xsum(a), ssh, bsh));
     const float gate = tab_dev ? tab_dev->shared_gate : tab_val.shared_gate;
     const float sum = __builtin_isnan(gate) ? moe + sh : __builtin_fmaf(sh, sigmoidf_ref(gate), moe);
     res = h_mid[row] + sum;
@@ -1008,65 +908,22 @@ __global__ __launch_bounds__(64) void k_down_combine(BlobGeom routed, BlobGeom s
   } else {
     res = h_mid[row] + moe;
   }
-  if (lch == 0 && valid) hidden_out[row] = res;
+  if (lane == 0) hidden_out[row] = res;
 }
 
-template <int BITS, int CPR, bool PAD = false>
-static hipError_t down_inst(const BlobGeom& routed, const BlobGeom& shared,
-                            const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t k,
-                            const float* act, const float* h_mid, const float* shared_out,
-                            float* hidden_out, hipStream_t st) {
-  constexpr int L = CPR < kWave ? CPR : kWave;
-  constexpr int RPP = kWave / L;
-  const uint32_t blocks = (routed.hidden + RPP - 1) / RPP;
-  if (k <= 8)
-    hipLaunchKernelGGL((k_down_combine<BITS, CPR, 8, PAD>), dim3(blocks), dim3(64), 0, st, routed,
-                       shared, tab_dev, tab_val, act, h_mid, shared_out, hidden_out);
+hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                               const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
+                               const float* shared_out, float* hidden_out, hipStream_t st) {
+  if (ph_down_supported(routed.inter, tab_val.k, n_slots > tab_val.k))
+    return launch_ph_down(routed, shared, tab_dev, tab_val, n_slots, act, h_mid, shared_out, hidden_out, st);
+  const uint32_t blocks = routed.hidden;
+  if (routed.bits == 4)
+    hipLaunchKernelGGL(k_down_combine<4>, dim3(blocks), dim3(64), 0, st, routed, shared, tab_dev, tab_val, act, h_mid,
+                       shared_out, hidden_out);
   else
-    hipLaunchKernelGGL((k_down_combine<BITS, CPR, 16, PAD>), dim3(blocks), dim3(64), 0, st, routed,
-                       shared, tab_dev, tab_val, act, h_mid, shared_out, hidden_out);
+    hipLaunchKernelGGL(k_down_combine<3>, dim3(blocks), dim3(64), 0, st, routed, shared, tab_dev, tab_val, act, h_mid,
+                       shared_out, hidden_out);
   return hipGetLastError();
-}
-
-template <int BITS>
-static hipError_t down_bits(const BlobGeom& routed, const BlobGeom& shared,
-                            const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t k,
-                            const float* act, const float* h_mid, const float* shared_out,
-                            float* hidden_out, hipStream_t st, bool* unsupported) {
-  const uint32_t cpr = routed.inter / kChunk;
-  switch (cpr) {
-    case 8: return down_inst<BITS, 8>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-    case 16: return down_inst<BITS, 16>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-    case 32: return down_inst<BITS, 32>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-    case 64: return down_inst<BITS, 64>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-    default: break;
-  }
-  // Other intermediate sizes (multiples of 32 up to 2048): the padded instances.
-  if (cpr == 0) {
-    *unsupported = true;
-    return hipSuccess;
-  }
-  if (cpr <= 2) return down_inst<BITS, 2, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  if (cpr <= 4) return down_inst<BITS, 4, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  if (cpr <= 8) return down_inst<BITS, 8, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  if (cpr <= 16) return down_inst<BITS, 16, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  if (cpr <= 32) return down_inst<BITS, 32, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  if (cpr <= 64) return down_inst<BITS, 64, true>(routed, shared, tab_dev, tab_val, k, act, h_mid, shared_out, hidden_out, st);
-  *unsupported = true;
-  return hipSuccess;
-}
-
-hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared,
-                               const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t n_slots,
-                               const float* act, const float* h_mid, const float* shared_out,
-                               float* hidden_out, hipStream_t st, bool* unsupported) {
-  *unsupported = false;
-  (void)n_slots;
-  const uint32_t k = tab_val.k;
-  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, act, h_mid,
-                                         shared_out, hidden_out, st, unsupported)
-                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, act, h_mid,
-                                         shared_out, hidden_out, st, unsupported);
 }
 
 // ---------------------------------------------------------------------------
@@ -1125,9 +982,7 @@ uint64_t prefill_tokens_workspace(uint32_t hidden, uint32_t inter, uint32_t n_to
 
 hipError_t launch_prefill_tokens(const BlobGeom& g, const uint8_t* experts, uint64_t stride, uint32_t E,
                                  const int32_t* idx, const float* w, const void* x, bool x_bf16, uint32_t n,
-                                 uint32_t k, float* out, uint8_t* ws, uint32_t* err, hipStream_t st,
-                                 bool* unsupported) {
-  *unsupported = false;
+                                 uint32_t k, float* out, uint8_t* ws, uint32_t* err, hipStream_t st) {
   auto al = [](uint64_t b) { return (b + 255) / 256 * 256; };
   FfnTable* tab = reinterpret_cast<FfnTable*>(ws);
   float* zero = reinterpret_cast<float*>(ws + al(sizeof(FfnTable)));
@@ -1144,10 +999,9 @@ hipError_t launch_prefill_tokens(const BlobGeom& g, const uint8_t* experts, uint
     hipLaunchKernelGGL(k_pt_table, dim3(1), dim3(64), 0, st, idx + (size_t)t * k, w + (size_t)t * k, k, E, experts,
                        stride, tab, err);
     e = hipGetLastError();
-    if (e == hipSuccess) e = launch_gateup(g, g, tab, tv, k, xf + (size_t)t * g.hidden, act, st, unsupported);
-    if (e == hipSuccess && !*unsupported)
-      e = launch_down_combine(g, g, tab, tv, k, act, zero, nullptr, out + (size_t)t * g.hidden, st, unsupported);
-    if (*unsupported) break;
+    if (e == hipSuccess) e = launch_gateup(g, g, tab, tv, k, xf + (size_t)t * g.hidden, act, st);
+    if (e == hipSuccess)
+      e = launch_down_combine(g, g, tab, tv, k, act, zero, nullptr, out + (size_t)t * g.hidden, st);
   }
   return e;
 }

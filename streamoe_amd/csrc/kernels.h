@@ -192,8 +192,7 @@ uint64_t prefill_workspace(uint32_t hidden, uint32_t inter, uint32_t group, uint
 uint64_t prefill_tokens_workspace(uint32_t hidden, uint32_t inter, uint32_t n_tokens, uint32_t k, bool x_bf16);
 hipError_t launch_prefill_tokens(const BlobGeom& g, const uint8_t* experts, uint64_t stride, uint32_t E,
                                  const int32_t* idx, const float* w, const void* x, bool x_bf16, uint32_t n,
-                                 uint32_t k, float* out, uint8_t* ws, uint32_t* err, hipStream_t st,
-                                 bool* unsupported);
+                                 uint32_t k, float* out, uint8_t* ws, uint32_t* err, hipStream_t st);
 // Prefill on the int8 matrix cores at f32 precision (limb.hip), for the same
 // shapes: every group size, hidden and inter multiples of 32, n * k entries
 // up to 65535.
@@ -263,12 +262,19 @@ hipError_t launch_noaux_topk(const float* logits, const float* bias, uint32_t n_
 // Exactly one of tab_dev / tab_val is used (tab_dev when not null).
 hipError_t launch_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                          const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act,
-                         hipStream_t st, bool* unsupported);
+                         hipStream_t st);
 // hidden_out = h_mid + sum_k w_k down_k(act_k) (+ shared term).
 hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared,
                                const FfnTable* tab_dev, const FfnTable& tab_val, uint32_t n_slots,
                                const float* act, const float* h_mid, const float* shared_out,
-                               float* hidden_out, hipStream_t st, bool* unsupported);
+                               float* hidden_out, hipStream_t st);
+// The same two steps with the activations as limbs in LDS (phase.hip).
+hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                            const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st);
+bool ph_down_supported(uint32_t inter, uint32_t k, bool has_shared);
+hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                          const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
+                          const float* shared_out, float* hidden_out, hipStream_t st);
 // Streaming-read diagnostic over `bytes` (multiple of 16) with
 // kStreamBlocks blocks; sink: kStreamBlocks u32.
 constexpr uint32_t kStreamBlocks = 2048;

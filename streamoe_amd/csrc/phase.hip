@@ -1,0 +1,416 @@
+// phase.hip — the expert FFN of one token as two kernels (gfx950), any width.
+//
+//   k_ph_gateup   gate + up + SwiGLU of every slot in the table (routed slots
+//                 and the shared expert).
+//   k_ph_down     down rows of every slot, combined in slot order with the
+//                 shared term and the residual.
+//
+// Both keep their activations (the hidden vector, the slots' SwiGLU outputs)
+// in LDS as 31-bit block floating point, one exponent per 32 values, in four
+// int8 limbs, written once per block while the weights are in flight: a
+// code then costs one byte unpack and four v_dot4c_i32_i8 per four inputs,
+// the sums are exact, and a chunk is rounded once, at f32 precision.
+// Converting codes to floats for FMAs, with every wave loading the
+// activations again, took 11.4 + 21.6 us per layer at 2560 x 640 (512 experts,
+// top-10, shared expert) and 6.4 + 8.7 at 2048 x 512 top-8; these take 10.5 +
+// 12.2 and 5.8 + 6.4: a launch, the table's and the rows' round trips and the
+// dots after them, at an eighth (2048 x 512) to half (7168 x 2048) of the HBM
+// rate.
+#include "common.h"
+#include "kernels.h"
+
+namespace smoe {
+
+constexpr int kL4Words = 36;  // LDS dwords per chunk: 32 of limbs, scale, sum, pad (conflict-free 16-byte reads)
+
+struct Limbs4 {
+  uint32_t w[4][8];
+  float scale, xs;
+};
+
+// A chunk's values as limbs, four lanes per chunk (lane q of the quad holds
+// values 8 q .. 8 q + 7): x_j = m_j 2^-f, |m_j| <= 2^30, bytes in the order of
+// unpack_bytes. live: store.
+__device__ __forceinline__ void store_limbs4_quad(uint32_t* dst, const float (&x)[8], int q, bool live) {
+  float amax = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
+  amax = fmaxf(amax, dpp_f<0xB1>(amax, 0.f));
+  amax = fmaxf(amax, dpp_f<0x4E>(amax, 0.f));
+  const int f = amax > 0.f ? 30 - __builtin_amdgcn_frexp_expf(amax) : 0;
+  int32_t d[4][8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int32_t m = (int32_t)__builtin_rintf(__builtin_ldexpf(x[j], f));
+    const int32_t d0 = (int32_t)((uint32_t)m << 24) >> 24, m1 = (m - d0) >> 8;
+    const int32_t d1 = (int32_t)((uint32_t)m1 << 24) >> 24, m2 = (m1 - d1) >> 8;
+    const int32_t d2 = (int32_t)((uint32_t)m2 << 24) >> 24;
+    d[0][j] = d0, d[1][j] = d1, d[2][j] = d2, d[3][j] = (m2 - d2) >> 8;
+  }
+  float xs = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  xs += dpp_f<0xB1>(xs, 0.f);
+  xs += dpp_f<0x4E>(xs, 0.f);
+  if (!live) return;
+#pragma unroll
+  for (int L = 0; L < 4; ++L)
+    *reinterpret_cast<uint2*>(dst + 8 * L + 2 * q) = make_uint2(
+        pack_bytes(d[L][0], d[L][2], d[L][4], d[L][6]), pack_bytes(d[L][1], d[L][3], d[L][5], d[L][7]));
+  if (q == 0) *reinterpret_cast<uint2*>(dst + 32) = make_uint2(__float_as_uint(__builtin_ldexpf(1.0f, -f)), __float_as_uint(xs));
+}
+
+__device__ __forceinline__ void load_limbs4(const uint32_t* p, Limbs4& o) {
+  const u32x4* p4 = reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u32x4 v = p4[i];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.w[i / 2][(i % 2) * 4 + c] = v[c];
+  }
+  const uint2 t = *reinterpret_cast<const uint2*>(p + 32);
+  o.scale = __uint_as_float(t.x);
+  o.xs = __uint_as_float(t.y);
+}
+
+// s * sum_j q_j x_j + b * sum_j x_j of one chunk.
+template <int BITS>
+__device__ __forceinline__ float chunk_dot4(const Raw<BITS>& raw, const Limbs4& x, float s, float b) {
+  uint32_t q[8];
+  unpack_bytes(raw, q);
+  int32_t S[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int w = 0; w < 8; ++w)
+#pragma unroll
+    for (int L = 0; L < 4; ++L) S[L] = __builtin_amdgcn_sdot4((int)q[w], (int)x.w[L][w], S[L], false);
+  // |S_L| <= 32 * 15 * 128: the pairs are exact in 32 bits and as floats.
+  const int32_t lo = S[0] + (int32_t)((uint32_t)S[1] << 8), hi = S[2] + (int32_t)((uint32_t)S[3] << 8);
+  return __builtin_fmaf(s, __builtin_fmaf((float)hi, 65536.f, (float)lo) * x.scale, b * x.xs);
+}
+
+// The blob of slot s and the table's scalars, from the device table or the
+// kernel argument (selects: a lane-indexed argument would go through
+// scratch).
+__device__ __forceinline__ const uint8_t* slot_blob(const FfnTable* dev, const FfnTable& val, uint32_t s) {
+  if (dev) return dev->blob[s];
+  const uint8_t* p = val.blob[0];
+#pragma unroll
+  for (uint32_t i = 1; i < (uint32_t)kMaxSlots; ++i) p = s == i ? val.blob[i] : p;
+  return p;
+}
+
+// ---------------------------------------------------------------------------
+// Gate/up. A wave takes 4 P rows (gate and up) of one slot: 16 lanes per row,
+// lane l the chunks l, l + 16, ..., IB of them per round (the last round's
+// past the row re-read its last chunk against zero limbs). 16 lanes per row
+// leave at most 15 of a row's chunk places empty, where whole-wave rows of
+// 80 chunks left 48 of 128.
+// ---------------------------------------------------------------------------
+template <int BITS, int P, int IB>
+__device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobGeom& g, uint32_t row0, uint32_t lane,
+                                               const float* x, uint32_t* limbs, float* act) {
+  constexpr int CB = chunk_bytes<BITS>();
+  const gbytes blob = as_global(blob_);
+  const uint32_t cpr = g.hidden / kChunk, gpr = g.hidden >> __builtin_ctz(g.group);
+  const uint32_t cps = __builtin_ctz(g.group / kChunk);
+  const uint32_t l16 = lane & 15, lrow = lane >> 4;
+  uint32_t row[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) row[p] = min(row0 + p * 4 + lrow, g.inter - 1);
+  Raw<BITS> raw[IB][P][2];
+  uint32_t sv[IB][P][2], bv[IB][P][2];
+  auto load = [&](uint32_t c0) {
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+      const uint32_t c = min(c0 + i * 16 + l16, cpr - 1);
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          raw[i][p][m] = load_raw_g<BITS>(blob + g.w[m] + (uint64_t)row[p] * (cpr * CB) + c * CB);
+          const uint64_t gi = ((uint64_t)row[p] * gpr + (c >> cps)) * 2;
+          sv[i][p][m] = gld<false, uint16_t>(blob + g.s[m] + gi);
+          bv[i][p][m] = gld<false, uint16_t>(blob + g.b[m] + gi);
+        }
+    }
+  };
+  load(0);
+  __builtin_amdgcn_sched_barrier(0);
+  // x as limbs: a quad of threads per chunk; chunks past the row are zero.
+  {
+    const uint32_t nq = blockDim.x >> 2, q = threadIdx.x & 3, padded = (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB);
+    for (uint32_t ch = threadIdx.x >> 2; ch < (padded + nq - 1) / nq * nq; ch += nq) {
+      const f32x4* const xp = reinterpret_cast<const f32x4*>(x + (size_t)min(ch, cpr - 1) * kChunk + q * 8);
+      f32x4 a = xp[0], b = xp[1];
+      if (ch >= cpr) a = b = f32x4{0.f, 0.f, 0.f, 0.f};
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      store_limbs4_quad(limbs + (size_t)min(ch, padded - 1) * kL4Words, v, (int)q, ch < padded);
+    }
+  }
+  // The block's limbs are written; the weights stay in flight.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  float sum[P][2];
+#pragma unroll
+  for (int p = 0; p < P; ++p) sum[p][0] = sum[p][1] = 0.f;
+  for (uint32_t c0 = 0;;) {
+#pragma unroll
+    for (int i = 0; i < IB; ++i) {
+      Limbs4 xl;
+      load_limbs4(limbs + (size_t)(c0 + i * 16 + l16) * kL4Words, xl);
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          sum[p][m] += chunk_dot4<BITS>(raw[i][p][m], xl, __uint_as_float(sv[i][p][m] << 16), __uint_as_float(bv[i][p][m] << 16));
+      __builtin_amdgcn_sched_barrier(0);  // one chunk's limbs in registers at a time
+    }
+    c0 += 16 * IB;
+    if (c0 >= cpr) break;
+    load(c0);
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const float gs = row_sum16_all(sum[p][0]), us = row_sum16_all(sum[p][1]);
+    const uint32_t r = row0 + p * 4 + lrow;
+    if (l16 == 0 && r < g.inter) act[r] = silu_mul(gs, us);
+  }
+}
+
+template <int BITS, int P, int IB, int WPB>
+__global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeom shared, const FfnTable* __restrict__ tab_dev,
+                                                        FfnTable tab_val, uint32_t tiles, const float* __restrict__ x,
+                                                        float* __restrict__ act) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (4 * P);
+  const uint32_t k = tab_dev ? tab_dev->k : tab_val.k;
+  const uint8_t* const blob = slot_blob(tab_dev, tab_val, slot);
+  float* const out = act + (size_t)slot * routed.inter;
+  if (slot < k)
+    ph_gateup_rows<BITS, P, IB>(blob, routed, row0, lane, x, lds, out);
+  else
+    ph_gateup_rows<4, P, IB>(blob, shared, row0, lane, x, lds, out);
+}
+
+// ---------------------------------------------------------------------------
+// Down + combine. One block per NR hidden rows (8; 4 in blocks of more
+// than 8 waves, whose lanes have half the registers); a lane owns one (slot,
+// chunk) of the flat list of k * inter / 32 and reads it for all the rows, so only
+// the last wave has empty lanes; one more wave takes the shared expert's
+// chunks (4-bit). The products go to LDS, a thread per (row, slot) adds a
+// slot's chunks, and a thread per row combines the slots in the reference's
+// order: moe = fma(out_s, w_s, moe) (deferred.rs:458-466), then the shared
+// term and the residual.
+// ---------------------------------------------------------------------------
+template <int BITS, bool NT, uint32_t NR>
+struct DownRows {
+  Raw<BITS> raw[NR];
+  uint32_t s[NR], b[NR];
+  __device__ __forceinline__ void load(const uint8_t* blob_, const BlobGeom& g, uint32_t row0, uint32_t c) {
+    const gbytes blob = as_global(blob_);
+    const uint32_t cpr = g.inter / kChunk, gpr = g.inter >> __builtin_ctz(g.group);
+    const uint32_t cg = c >> __builtin_ctz(g.group / kChunk);
+#pragma unroll
+    for (uint32_t r = 0; r < NR; ++r) {
+      const uint32_t row = min(row0 + r, g.hidden - 1);
+      raw[r] = load_raw_g<BITS, NT>(blob + g.w[2] + (uint64_t)row * (cpr * chunk_bytes<BITS>()) + c * chunk_bytes<BITS>());
+      const uint64_t gi = ((uint64_t)row * gpr + cg) * 2;
+      s[r] = gld<false, uint16_t>(blob + g.s[2] + gi);
+      b[r] = gld<false, uint16_t>(blob + g.b[2] + gi);
+    }
+  }
+  __device__ __forceinline__ void dot(const uint32_t* limbs, float* part, uint32_t ld) const {
+    Limbs4 xl;
+    load_limbs4(limbs, xl);
+#pragma unroll
+    for (uint32_t r = 0; r < NR; ++r)
+      part[r * ld] = chunk_dot4<BITS>(raw[r], xl, __uint_as_float(s[r] << 16), __uint_as_float(b[r] << 16));
+  }
+};
+
+// LDS of k_ph_down: limbs of every chunk, then the products [NR][ld].
+__host__ __device__ constexpr uint32_t ph_down_ld(uint32_t chunks) { return chunks | 1u; }
+__host__ __device__ constexpr uint32_t ph_down_lds(uint32_t chunks, uint32_t nr) {
+  return chunks * kL4Words * 4 + nr * ph_down_ld(chunks) * 4;
+}
+
+template <int BITS, uint32_t NR, int TB>
+__global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared, const FfnTable* __restrict__ tab_dev,
+                                                  FfnTable tab_val, uint32_t k, uint32_t has_shared,
+                                                  const float* __restrict__ act, const float* h_mid,
+                                                  const float* __restrict__ shared_out, float* hidden_out) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ float so[NR][kMaxSlots + 1];
+  __shared__ float sw[kMaxSlots];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t I = routed.inter, H = routed.hidden, cpr = I / kChunk;
+  const uint32_t items = k * cpr, chunks = (k + has_shared) * cpr, ld = ph_down_ld(chunks);
+  const uint32_t rwaves = (blockDim.x >> 6) - has_shared;
+  const uint32_t row0 = blockIdx.x * NR;
+  const bool is_routed = wave < rwaves;
+  const uint32_t item = is_routed ? min(wave * 64 + lane, items - 1) : items + min(lane, cpr - 1);
+  const uint32_t slot = item / cpr, c = item - slot * cpr;
+  const uint8_t* const blob = slot_blob(tab_dev, tab_val, slot);
+  // What the combine needs, ahead of the weights.
+  float hm = 0.f, sh_in = 0.f, gate = 0.f, wk = 0.f;
+  if (tid < NR) {
+    const uint32_t r = min(row0 + tid, H - 1);
+    hm = h_mid[r];
+    gate = tab_dev ? tab_dev->shared_gate : tab_val.shared_gate;
+    if (!has_shared && shared_out) sh_in = shared_out[r];
+  }
+  if (tab_dev) {
+    if (tid < k) wk = tab_dev->weight[tid];
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)kMaxK; ++i) wk = tid == i ? tab_val.weight[i] : wk;
+  }
+  // Activations: a quad of threads per chunk, at most four rounds (64 lanes
+  // per wave hold 16 quads, and there is a lane per chunk).
+  const uint32_t nq = blockDim.x >> 2, qd = tid >> 2, q = tid & 3;
+  f32x4 st[4][2];
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const f32x4* const p = reinterpret_cast<const f32x4*>(act + (size_t)min(qd + i * nq, chunks - 1) * kChunk + q * 8);
+    st[i][0] = p[0];
+    st[i][1] = p[1];
+  }
+  uint32_t* const limbs = lds;
+  float* const part = reinterpret_cast<float*>(lds + (size_t)chunks * kL4Words);
+  auto stage = [&]() {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      if (i * nq >= chunks) break;
+      const uint32_t ch = qd + i * nq;
+      const float v[8] = {st[i][0].x, st[i][0].y, st[i][0].z, st[i][0].w, st[i][1].x, st[i][1].y, st[i][1].z, st[i][1].w};
+      store_limbs4_quad(limbs + (size_t)min(ch, chunks - 1) * kL4Words, v, (int)q, ch < chunks);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (is_routed) {
+    DownRows<BITS, true, NR> d;
+    d.load(blob, routed, row0, c);
+    __builtin_amdgcn_sched_barrier(0);
+    stage();
+    if (wave * 64 + lane < items) d.dot(limbs + (size_t)item * kL4Words, part + item, ld);
+  } else {
+    DownRows<4, false, NR> d;
+    d.load(blob, shared, row0, c);
+    __builtin_amdgcn_sched_barrier(0);
+    stage();
+    if (lane < cpr) d.dot(limbs + (size_t)item * kL4Words, part + item, ld);
+  }
+  if (tid < k) sw[tid] = wk;
+  __syncthreads();
+  // Thread (row, slot): the slot's chunks in four interleaved sums.
+  for (uint32_t i = tid; i < NR * (k + has_shared); i += blockDim.x) {
+    const uint32_t r = i % NR, s = i / NR;
+    const float* const p = part + r * ld + s * cpr;
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    uint32_t j = 0;
+    for (; j + 4 <= cpr; j += 4)
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) a[v] += p[j + v];
+    for (; j < cpr; ++j) a[j & 3] += p[j];
+    so[r][s] = (a[0] + a[1]) + (a[2] + a[3]);
+  }
+  __syncthreads();
+  if (tid < NR && row0 + tid < H) {
+    float moe = 0.f;
+    for (uint32_t s = 0; s < k; ++s) moe = __builtin_fmaf(so[tid][s], sw[s], moe);
+    float sum = moe;
+    if (has_shared || shared_out) {
+      const float sh = has_shared ? so[tid][k] : sh_in;
+      sum = __builtin_isnan(gate) ? moe + sh : __builtin_fmaf(sh, sigmoidf_ref(gate), moe);
+    }
+    hidden_out[row0 + tid] = hm + sum;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Host side.
+// ---------------------------------------------------------------------------
+template <int BITS, int P, int IB, int WPB>
+static hipError_t gateup_inst(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  const uint32_t tiles = (routed.inter + 4 * P * WPB - 1) / (4 * P * WPB);
+  const uint32_t cpr = routed.hidden / kChunk, padded = (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB);
+  hipLaunchKernelGGL((k_ph_gateup<BITS, P, IB, WPB>), dim3(tiles * n_slots), dim3(64 * WPB), padded * kL4Words * 4, st,
+                     routed, shared, tab_dev, tab_val, tiles, x, act);
+  return hipGetLastError();
+}
+
+template <int BITS, int P>
+static hipError_t gateup_rows(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  // Rounds of 5 chunks per lane where they divide the row into fewer places
+  // than rounds of 4 (2560: one of 5, not two of 4).
+  const uint32_t n = (routed.hidden / kChunk + 15) / 16;
+  if (n == 1) return gateup_inst<BITS, P, 1, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+  if ((n + 4) / 5 * 5 < (n + 3) / 4 * 4) return gateup_inst<BITS, P, 5, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+  return gateup_inst<BITS, P, 4, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+}
+
+template <int BITS>
+static hipError_t gateup_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  // 4 rows per wave while that makes no more than 1024 waves (one per SIMD),
+  // else 8, whose limbs serve two rows each: 8 slots of 2048 x 512 (gate/up
+  // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
+  // 2560 x 640 18.8 against 17.3, 8 of 7168 x 2048 74.0 against 72.2. Four
+  // waves share a block's limbs (one: 12.2, two: 11.3 at 2048 x 512).
+  if (n_slots * routed.inter <= 4096) return gateup_rows<BITS, 1>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+  return gateup_rows<BITS, 2>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+}
+
+hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                            const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  return routed.bits == 4 ? gateup_bits<4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st)
+                          : gateup_bits<3>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+}
+
+// Waves of a k_ph_down block: a lane per (slot, chunk), and the shared wave.
+static uint32_t ph_down_waves(uint32_t inter, uint32_t k, bool has_shared) {
+  return (k * (inter / kChunk) + 63) / 64 + has_shared;
+}
+constexpr uint32_t kPdLds = 156 * 1024;
+bool ph_down_supported(uint32_t inter, uint32_t k, bool has_shared) {
+  return ph_down_waves(inter, k, has_shared) <= 16 && ph_down_lds((k + has_shared) * (inter / kChunk), 4) <= kPdLds;
+}
+
+template <int BITS, uint32_t NR, int TB>
+static hipError_t down_inst(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                            const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
+                            const float* h_mid, const float* shared_out, float* hidden_out, hipStream_t st) {
+  const uint32_t lds = ph_down_lds((k + has_shared) * (routed.inter / kChunk), NR);
+  if (lds > 60 * 1024) {
+    static std::atomic<uint64_t> raised{0};
+    const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_ph_down<BITS, NR, TB>), kPdLds, raised);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_ph_down<BITS, NR, TB>), dim3((routed.hidden + NR - 1) / NR),
+                     dim3(64 * ph_down_waves(routed.inter, k, has_shared)), lds, st, routed, shared, tab_dev, tab_val, k,
+                     has_shared, act, h_mid, shared_out, hidden_out);
+  return hipGetLastError();
+}
+
+template <int BITS>
+static hipError_t down_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                            const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
+                            const float* h_mid, const float* shared_out, float* hidden_out, hipStream_t st) {
+  if (ph_down_waves(routed.inter, k, has_shared) <= 8)
+    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
+  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
+}
+
+hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                          const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
+                          const float* shared_out, float* hidden_out, hipStream_t st) {
+  const uint32_t k = tab_val.k, has_shared = n_slots > k ? 1u : 0u;
+  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st)
+                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
+}
+
+}  // namespace smoe

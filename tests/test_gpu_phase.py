@@ -1,0 +1,76 @@
+"""The one-token expert kernels with limbs in LDS (csrc/phase.hip) at the edges
+of their tiles and of the rules that choose between kernels, against the
+oracle. Bar: max|d| / max|ref| <= 1e-5 of the output and of the MoE part: the
+oracle's sequential f32 sums of K <= 8128 terms are off by about sqrt(K) 2^-24,
+5.4e-6, the device's by less."""
+import numpy as np
+import pytest
+
+from helpers import rel_err
+from test_gpu_decode import _experts_case, _layer_case, _torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+@pytest.mark.parametrize("H,I,k,bits,shared", [
+    (64, 64, 1, 4, False),      # two chunks: a sixteenth of a row's lanes
+    (576, 192, 3, 3, True),     # 18 chunks: one round of four, two of them used
+    (2048, 448, 9, 4, False),   # 4032 rows: 4 per wave
+    (2048, 576, 8, 4, True),    # 4608 rows: 8 per wave
+    (2624, 704, 7, 3, True),    # 82 chunks: two rounds of four; three waves of 8 down rows
+    (2560, 1600, 10, 4, True),  # 8 down waves
+    (2560, 1664, 10, 4, True),  # 9: half the rows per block
+    (8128, 128, 2, 4, False),   # 254 chunks
+    (4096, 320, 4, 3, True),    # hidden 4096: whole-wave gate/up rows
+    (128, 1984, 16, 4, True),   # 992 chunks, the most that fit
+    (128, 2048, 16, 3, True),   # 1024: a wave per row
+])
+def test_phase_experts_match_oracle(kernels, H, I, k, bits, shared):
+    if H > 4096:
+        kernels.reserve(H, 2048, 1024)
+    got, want, h_mid = _experts_case(kernels, H, I, k, bits, shared, seed=H + I + k + bits)
+    err, moe = rel_err(got, want), rel_err(got - h_mid, want - h_mid)
+    print(f"experts H={H} I={I} k={k} {bits}-bit rel_err={err:.3e} MoE part {moe:.3e}")
+    assert err <= TOL and moe <= TOL
+
+
+@pytest.mark.parametrize("name,H,I,E,k,bits,shared", [
+    ("small-3bit", 320, 192, 20, 5, 3, True),   # 3-bit routed slots beside the 4-bit shared wave
+    ("ungated", 2560, 640, 40, 10, 4, "ungated"),
+    ("most-chunks", 256, 1856, 18, 16, 4, True),   # 17 slots, 986 chunks
+    ("wave-per-row", 256, 1920, 18, 16, 3, True),  # 1020
+])
+def test_phase_layers_match_oracle(kernels, name, H, I, E, k, bits, shared):
+    kernels.set_decode_path(1)
+    try:
+        got, gi, gw, want, wi, ww, _ = _layer_case(kernels, H, I, E, k, bits, True, shared, seed=sum(map(ord, name)))
+    finally:
+        kernels.set_decode_path(0)
+    kernels.sync()
+    err = rel_err(got, want)
+    print(f"layer {name}: rel_err={err:.3e}")
+    assert np.array_equal(gi, wi)
+    assert err <= TOL
+
+
+def test_phase_nonfinite_input(kernels):
+    """A NaN in the hidden vector reaches every output; the next call is clean."""
+    import streamoe_amd as sa
+
+    torch = _torch()
+    lay = sa.ExpertLayout(576, 192, 4, 64)
+    arena = torch.empty(2 * lay.expert_size, dtype=torch.uint8, device="cuda")
+    assert kernels.synth_experts(arena, 2, lay.expert_size, lay, 3) == 0
+    x = torch.ones(576, device="cuda")
+    out, h = torch.empty(576, device="cuda"), torch.zeros(576, device="cuda")
+    bind = [(arena, 0), (arena, lay.expert_size)]
+    x[100] = float("nan")
+    assert kernels.experts_decode(lay, bind, [0.5, 0.5], x, h, None, 0.0, out) == 0
+    kernels.sync()
+    assert bool(torch.isnan(out).all())
+    x[100] = 1.0
+    assert kernels.experts_decode(lay, bind, [0.5, 0.5], x, h, None, 0.0, out) == 0
+    kernels.sync()
+    assert bool(torch.isfinite(out).all())
