@@ -56,15 +56,28 @@ __device__ __forceinline__ void softmax_ref(float (&v)[P], uint32_t n, int lane,
   }
   __syncthreads();
   // Sequential sum in index order; the zeros past n change nothing (the sum
-  // of non-negative values is never -0).
+  // of non-negative values is never -0). 32 values per round, the next
+  // round's LDS reads under way during a round's additions (a read waited for
+  // every four additions cost 1.2 us at 512
+  // experts).
   float sum = 0.f;
   const f32x4* s4 = reinterpret_cast<const f32x4*>(sbuf);
-  for (uint32_t i = 0; i < (n + 3) / 4; ++i) {
-    const f32x4 q = s4[i];
-    sum += q.x;
-    sum += q.y;
-    sum += q.z;
-    sum += q.w;
+  f32x4 cur[8], nxt[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) cur[j] = s4[j];
+#pragma unroll
+  for (int r = 0; r < 2 * P; ++r) {
+    if (r + 1 < 2 * P) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) nxt[j] = s4[(r + 1) * 8 + j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sum += cur[j][c];
+    if ((uint32_t)(r + 1) * 32 >= n) break;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) cur[j] = nxt[j];
   }
   const float inv = __fdiv_rn(1.0f, sum);
 #pragma unroll
@@ -187,14 +200,30 @@ __device__ void exact_topk(const float (&v)[P], uint32_t k, int lane, int32_t* o
 // be null.
 template <int P>
 __device__ int32_t exact_topk_t(const float (&v)[P], uint32_t k, int lane, int32_t* out_idx, float* out_val) {
-  uint64_t key = lane < (int)k ? (((uint64_t)orderable(-1e30f) << 32) | (uint32_t)lane) : ~0ull;
-  int32_t qidx = 0;
+  // Queue entry per lane q < k, sorted by (value, slot): the value, and slot
+  // << 16 | element index (at most 1024 elements).
   float qval = -1e30f;
+  uint32_t qent = (uint32_t)lane << 16;
   // Queue lanes 1 .. k-1 (k <= 64): where a new entry may be placed.
   const uint64_t qmask = (k >= 64 ? ~0ull : ((1ull << k) - 1)) & ~1ull;
+  // The first k elements take slots 0 .. k-1 one after another when they all
+  // beat the start value: sorted at once instead of k replacements.
+  uint32_t taken = 0;
+  const uint64_t live = qmask | 1ull;
+  if (k < 64 && (__ballot(v[0] > -1e30f) & live) == live) {
+    uint32_t rank = 0;
+    for (uint32_t r = 0; r < k; ++r) {
+      const float o = readlane_f(v[0], (int)r);
+      rank += (o < v[0] || (o == v[0] && (int)r < lane)) ? 1u : 0u;
+    }
+    const int dst = lane < (int)k ? (int)rank * 4 : lane * 4;
+    qval = __int_as_float(__builtin_amdgcn_ds_permute(dst, __float_as_int(v[0])));
+    qent = (uint32_t)__builtin_amdgcn_ds_permute(dst, (lane << 16) | lane);
+    taken = k;
+  }
 #pragma unroll
   for (int e = 0; e < P; ++e) {
-    uint64_t pend = ~0ull;  // lanes of chunk e not yet passed
+    uint64_t pend = e == 0 ? ~0ull << taken : ~0ull;  // lanes of chunk e not yet passed
     for (int guard = 0; guard < 64; ++guard) {
       const float hval = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(qval)));
       const uint64_t hit = __ballot(v[e] > hval) & pend;
@@ -202,25 +231,23 @@ __device__ int32_t exact_topk_t(const float (&v)[P], uint32_t k, int lane, int32
       const int first = __builtin_ctzll(hit);
       pend = first == 63 ? 0ull : pend & (~0ull << (first + 1));
       const float pj = readlane_f(v[e], first);
-      const uint32_t hslot = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)key);
-      const uint64_t nkey = ((uint64_t)orderable(pj) << 32) | hslot;
-      const int p = __popcll(__ballot(key < nkey) & qmask);  // new position among the k
-      const uint64_t kn = ((uint64_t)wave_next_u32((uint32_t)(key >> 32)) << 32) | wave_next_u32((uint32_t)key);
-      const int32_t in = (int32_t)wave_next_u32((uint32_t)qidx);
+      const uint32_t hslot = (uint32_t)__builtin_amdgcn_readfirstlane((int)qent) & 0xFFFF0000u;
+      // New position among the k: the entries below (pj, slot).
+      const int p = __popcll((__ballot(qval < pj) | (__ballot(qval == pj) & __ballot(qent < hslot))) & qmask);
+      const uint32_t en = wave_next_u32(qent);
       const float vn = __uint_as_float(wave_next_u32(__float_as_uint(qval)));
       // Lane q < p takes lane q+1's entry, lane p the new one (selects).
       const bool sh = lane < p, at = lane == p;
-      key = sh ? kn : (at ? nkey : key);
-      qidx = sh ? in : (at ? e * 64 + first : qidx);
+      qent = sh ? en : (at ? hslot | (uint32_t)(e * 64 + first) : qent);
       qval = sh ? vn : (at ? pj : qval);
     }
   }
   if (lane < (int)k) {
-    const uint32_t slot = (uint32_t)key;
-    if (out_idx) out_idx[slot] = qidx;
+    const uint32_t slot = qent >> 16;
+    if (out_idx) out_idx[slot] = (int32_t)(qent & 0xFFFFu);
     if (out_val) out_val[slot] = qval;
   }
-  return lane < (int)k ? qidx : -1;
+  return lane < (int)k ? (int32_t)(qent & 0xFFFFu) : -1;
 }
 
 // Bitwise OR over the wave, valid in lane 63 (DPP row shifts, then the
