@@ -564,13 +564,18 @@ static int decode_layer(smoe_handle* h, const smoe_layer* L, const float* input,
   ro.stride = L->stride;
   ro.shared_blob = (const uint8_t*)L->shared_expert;
   ro.gate_scores = (L->shared_expert && (L->shared_gate || L->shared_gate_q)) ? h->gate : nullptr;
-  e = launch_topk(h->logits, 1, L->n_experts, L->k, true, L->normalize != 0, ro, h->stream);
-  if (e != hipSuccess) return SMOE_ERR_HIP;
   const BlobGeom g = blob_geom(s.hidden, s.inter, s.group, s.bits);
   const BlobGeom gs = blob_geom(s.hidden, s.inter, s.group, 4);
   FfnTable tv{};
   tv.k = L->k;
   const uint32_t n_slots = L->k + (L->shared_expert ? 1 : 0);
+  if (ph_route_supported(s.hidden, L->n_experts) && ph_down_supported(s.inter, L->k, n_slots > L->k)) {
+    e = launch_ph_route(g, gs, h->logits, L->n_experts, L->k, L->normalize != 0, ro, n_slots, input, h->act, h->stream);
+    if (e != hipSuccess) return SMOE_ERR_HIP;
+    return hip_status(launch_ph_down(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out, h->stream, true));
+  }
+  e = launch_topk(h->logits, 1, L->n_experts, L->k, true, L->normalize != 0, ro, h->stream);
+  if (e != hipSuccess) return SMOE_ERR_HIP;
   e = launch_gateup(g, gs, h->table, tv, n_slots, input, h->act, h->stream);
   if (e != hipSuccess) return SMOE_ERR_HIP;
   e = launch_down_combine(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out, h->stream);

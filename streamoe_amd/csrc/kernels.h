@@ -47,6 +47,7 @@ struct FfnTable {
   float shared_gate;  // NaN: add the shared output unscaled
   uint32_t k;
   uint32_t has_shared;
+  uint8_t order[kMaxKHost];  // place of the reference's slot s in this table (k_ph_route only)
 };
 
 // Routing destination for the top-k kernel in layer mode.
@@ -271,10 +272,17 @@ hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared,
 // The same two steps with the activations as limbs in LDS (phase.hip).
 hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st);
+// The routing (from the logits, at least 64 P floats readable, P = 4 or 8) and
+// the gate/up step in one launch; the table's slots are then in its own
+// order, so the down step has to take table.order (ordered).
+bool ph_route_supported(uint32_t hidden, uint32_t n_experts);
+hipError_t launch_ph_route(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t n_experts,
+                           uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
+                           float* act, hipStream_t st);
 bool ph_down_supported(uint32_t inter, uint32_t k, bool has_shared);
 hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                           const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
-                          const float* shared_out, float* hidden_out, hipStream_t st);
+                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered = false);
 // Streaming-read diagnostic over `bytes` (multiple of 16) with
 // kStreamBlocks blocks; sink: kStreamBlocks u32.
 constexpr uint32_t kStreamBlocks = 2048;

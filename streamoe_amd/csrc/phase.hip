@@ -2,6 +2,7 @@
 //
 //   k_ph_gateup   gate + up + SwiGLU of every slot in the table (routed slots
 //                 and the shared expert).
+//   k_ph_route    the same with the routing in the launch.
 //   k_ph_down     down rows of every slot, combined in slot order with the
 //                 shared term and the residual.
 //
@@ -16,8 +17,11 @@
 // 12.2 and 5.8 + 6.4: a launch, the table's and the rows' round trips and the
 // dots after them, at an eighth (2048 x 512) to half (7168 x 2048) of the HBM
 // rate.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
+#include "topk.h"
 
 namespace smoe {
 
@@ -104,7 +108,21 @@ __device__ __forceinline__ const uint8_t* slot_blob(const FfnTable* dev, const F
 // leave at most 15 of a row's chunk places empty, where whole-wave rows of
 // 80 chunks left 48 of 128.
 // ---------------------------------------------------------------------------
-template <int BITS, int P, int IB>
+// x as limbs: a quad of threads per chunk; chunks past the row are zero.
+template <int IB>
+__device__ __forceinline__ void stage_x(const float* x, uint32_t cpr, uint32_t* limbs) {
+  const uint32_t nq = blockDim.x >> 2, q = threadIdx.x & 3, padded = (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB);
+  for (uint32_t ch = threadIdx.x >> 2; ch < (padded + nq - 1) / nq * nq; ch += nq) {
+    const f32x4* const xp = reinterpret_cast<const f32x4*>(x + (size_t)min(ch, cpr - 1) * kChunk + q * 8);
+    f32x4 a = xp[0], b = xp[1];
+    if (ch >= cpr) a = b = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    store_limbs4_quad(limbs + (size_t)min(ch, padded - 1) * kL4Words, v, (int)q, ch < padded);
+  }
+}
+
+// STAGE: the limbs are still to be written (after the weights' loads).
+template <int BITS, int P, int IB, bool STAGE>
 __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobGeom& g, uint32_t row0, uint32_t lane,
                                                const float* x, uint32_t* limbs, float* act) {
   constexpr int CB = chunk_bytes<BITS>();
@@ -134,17 +152,7 @@ __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobG
   };
   load(0);
   __builtin_amdgcn_sched_barrier(0);
-  // x as limbs: a quad of threads per chunk; chunks past the row are zero.
-  {
-    const uint32_t nq = blockDim.x >> 2, q = threadIdx.x & 3, padded = (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB);
-    for (uint32_t ch = threadIdx.x >> 2; ch < (padded + nq - 1) / nq * nq; ch += nq) {
-      const f32x4* const xp = reinterpret_cast<const f32x4*>(x + (size_t)min(ch, cpr - 1) * kChunk + q * 8);
-      f32x4 a = xp[0], b = xp[1];
-      if (ch >= cpr) a = b = f32x4{0.f, 0.f, 0.f, 0.f};
-      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      store_limbs4_quad(limbs + (size_t)min(ch, padded - 1) * kL4Words, v, (int)q, ch < padded);
-    }
-  }
+  if constexpr (STAGE) stage_x<IB>(x, cpr, limbs);
   // The block's limbs are written; the weights stay in flight.
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -187,9 +195,121 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeo
   const uint8_t* const blob = slot_blob(tab_dev, tab_val, slot);
   float* const out = act + (size_t)slot * routed.inter;
   if (slot < k)
-    ph_gateup_rows<BITS, P, IB>(blob, routed, row0, lane, x, lds, out);
+    ph_gateup_rows<BITS, P, IB, true>(blob, routed, row0, lane, x, lds, out);
   else
-    ph_gateup_rows<4, P, IB>(blob, shared, row0, lane, x, lds, out);
+    ph_gateup_rows<4, P, IB, true>(blob, shared, row0, lane, x, lds, out);
+}
+
+// ---------------------------------------------------------------------------
+// Routing and gate/up in one launch. Every routed wave takes its slot's expert
+// itself, the slot-th member of the top-k set in ascending index order
+// (topk_slot_logits: softmax is monotone, so the set is that of the logits
+// where the margin is clear; else the reference's probabilities and scan).
+// The last block finds the reference's slot order and weights, as k_topk
+// does, while the others stream their rows: at 512 experts, top-10, its 11 us
+// were a launch of their own between the router and the experts (39 -> 32 us
+// per layer at 2560 x 640). It writes the table in the order the
+// act rows have, and the place of each of the reference's slots in it.
+// ---------------------------------------------------------------------------
+template <int PL>
+struct RouteLds {
+  float prob[64 * PL];
+  float val[kMaxK];
+  int32_t id[kMaxK], set[kMaxK];
+  int32_t is_set;
+};
+
+template <int PL>
+__device__ void ph_route_table(const float* __restrict__ logits, uint32_t E, uint32_t k, int normalize,
+                               const RouteOut& out, uint32_t wave, int lane, RouteLds<PL>& s) {
+  float v[PL], l[PL];
+#pragma unroll
+  for (int e = 0; e < PL; ++e) {
+    const uint32_t jt = e * 64 + lane, jl = lane * PL + e;
+    v[e] = jt < E ? logits[jt] : -INFINITY;
+    l[e] = jl < E ? logits[jl] : -INFINITY;
+  }
+  // The set on a wave of its own beside the scan (the other waves only meet
+  // the barriers: three in softmax_ref, one after the scan).
+  if (wave != 0) {
+    if (wave == 1) {
+      const bool set = topk_set_logits<PL>(l, E, k, lane, s.set);
+      if (lane == 0) s.is_set = set;
+    }
+    for (int i = 0; i < 4; ++i) __syncthreads();
+    return;
+  }
+  softmax_ref<PL, true>(v, E, lane, s.prob, load_exp_tab(lane));
+  exact_topk_t<PL>(v, k, lane, s.id, s.val);
+  __syncthreads();
+  const int32_t id = lane < (int)k ? s.id[lane] : 0;
+  const float sv = lane < (int)k ? s.val[lane] : 0.f;
+  // normalize_weights, moe_router.rs:130-141: sequential sum in slot order.
+  float w = sv;
+  if (normalize) {
+    float sum = 0.f;
+    for (uint32_t i = 0; i < k; ++i) sum += readlane_f(sv, (int)i);
+    if (sum > 0.f) w = sv * (1.0f / sum);
+  }
+  const bool is_set = s.is_set;
+  uint32_t at = is_set ? 0u : (uint32_t)lane;  // place among the ascending indices
+  if (is_set)
+    for (uint32_t i = 0; i < k; ++i) at += s.set[i] < id ? 1u : 0u;
+  if (lane >= (int)k) return;
+  if (out.idx) out.idx[lane] = id;
+  if (out.weight) out.weight[lane] = w;
+  out.table->blob[at] = out.experts + (uint64_t)id * out.stride;
+  out.table->weight[at] = w;
+  out.table->order[lane] = (uint8_t)at;
+  if (lane == 0) {
+    out.table->k = k;
+    out.table->has_shared = out.shared_blob != nullptr;
+    if (out.shared_blob) {
+      out.table->blob[k] = out.shared_blob;
+      out.table->weight[k] = 1.0f;
+      out.table->shared_gate = out.gate_scores ? out.gate_scores[0] : __builtin_nanf("");
+    }
+  }
+}
+
+template <int BITS, int PL, int P, int IB, int WPB>
+__global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom shared, const float* __restrict__ logits,
+                                                       uint32_t E, uint32_t k, int normalize, RouteOut ro, uint32_t tiles,
+                                                       const float* __restrict__ x, float* __restrict__ act) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ RouteLds<PL> rl[WPB];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (4 * P);
+  // Every wave of a block goes the same way (they read the same logits), so
+  // the barriers inside are met by all of them.
+  if (blockIdx.x == gridDim.x - 1) {
+    ph_route_table<PL>(logits, E, k, normalize, ro, wave, (int)lane, rl[0]);
+    return;
+  }
+  float* const out = act + (size_t)slot * routed.inter;
+  if (slot == k) {
+    ph_gateup_rows<4, P, IB, true>(ro.shared_blob, shared, row0, lane, x, lds, out);
+    return;
+  }
+  float l[PL];
+#pragma unroll
+  for (int e = 0; e < PL / 4; ++e) {
+    const f32x4 q = *reinterpret_cast<const f32x4*>(logits + lane * PL + 4 * e);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) l[4 * e + c] = lane * PL + 4 * e + c < E ? q[c] : -INFINITY;
+  }
+  stage_x<IB>(x, routed.hidden / kChunk, lds);
+  int32_t id;
+  if (!topk_slot_logits<PL>(l, E, k, slot, (int)lane, id)) {
+    float v[PL];
+#pragma unroll
+    for (int e = 0; e < PL; ++e) v[e] = e * 64 + lane < E ? logits[e * 64 + lane] : -INFINITY;
+    softmax_ref<PL, true>(v, E, (int)lane, rl[wave].prob, load_exp_tab((int)lane));
+    exact_topk_t<PL>(v, k, (int)lane, rl[wave].id, nullptr);
+    __syncthreads();
+    id = __builtin_amdgcn_readfirstlane(rl[wave].id[slot]);
+  }
+  ph_gateup_rows<BITS, P, IB, false>(ro.experts + (uint64_t)id * ro.stride, routed, row0, lane, x, lds, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -238,8 +358,10 @@ template <int BITS, uint32_t NR, int TB>
 __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared, const FfnTable* __restrict__ tab_dev,
                                                   FfnTable tab_val, uint32_t k, uint32_t has_shared,
                                                   const float* __restrict__ act, const float* h_mid,
-                                                  const float* __restrict__ shared_out, float* hidden_out) {
+                                                  const float* __restrict__ shared_out, float* hidden_out,
+                                                  int ordered) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ uint8_t sord[kMaxK];
   __shared__ float so[NR][kMaxSlots + 1];
   __shared__ float sw[kMaxSlots];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -261,7 +383,9 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
   }
   if (tab_dev) {
     if (tid < k) wk = tab_dev->weight[tid];
+    if (tid < k) sord[tid] = ordered ? tab_dev->order[tid] : (uint8_t)tid;
   } else {
+    if (tid < k) sord[tid] = (uint8_t)tid;
 #pragma unroll
     for (uint32_t i = 0; i < (uint32_t)kMaxK; ++i) wk = tid == i ? tab_val.weight[i] : wk;
   }
@@ -319,7 +443,10 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
   __syncthreads();
   if (tid < NR && row0 + tid < H) {
     float moe = 0.f;
-    for (uint32_t s = 0; s < k; ++s) moe = __builtin_fmaf(so[tid][s], sw[s], moe);
+    for (uint32_t i = 0; i < k; ++i) {
+      const uint32_t s = sord[i];
+      moe = __builtin_fmaf(so[tid][s], sw[s], moe);
+    }
     float sum = moe;
     if (has_shared || shared_out) {
       const float sh = has_shared ? so[tid][k] : sh_in;
@@ -332,37 +459,67 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
-template <int BITS, int P, int IB, int WPB>
-static hipError_t gateup_inst(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
-                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
-  const uint32_t tiles = (routed.inter + 4 * P * WPB - 1) / (4 * P * WPB);
-  const uint32_t cpr = routed.hidden / kChunk, padded = (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB);
-  hipLaunchKernelGGL((k_ph_gateup<BITS, P, IB, WPB>), dim3(tiles * n_slots), dim3(64 * WPB), padded * kL4Words * 4, st,
-                     routed, shared, tab_dev, tab_val, tiles, x, act);
-  return hipGetLastError();
-}
-
-template <int BITS, int P>
-static hipError_t gateup_rows(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
-                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
-  // Rounds of 5 chunks per lane where they divide the row into fewer places
-  // than rounds of 4 (2560: one of 5, not two of 4).
-  const uint32_t n = (routed.hidden / kChunk + 15) / 16;
-  if (n == 1) return gateup_inst<BITS, P, 1, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  if ((n + 4) / 5 * 5 < (n + 3) / 4 * 4) return gateup_inst<BITS, P, 5, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  return gateup_inst<BITS, P, 4, 4>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-}
-
-template <int BITS>
-static hipError_t gateup_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
-                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+// Calls fn with the instance's (P, IB) as integral constants.
+template <typename F>
+static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {
   // 4 rows per wave while that makes no more than 1024 waves (one per SIMD),
   // else 8, whose limbs serve two rows each: 8 slots of 2048 x 512 (gate/up
   // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
   // 2560 x 640 18.8 against 17.3, 8 of 7168 x 2048 74.0 against 72.2. Four
   // waves share a block's limbs (one: 12.2, two: 11.3 at 2048 x 512).
-  if (n_slots * routed.inter <= 4096) return gateup_rows<BITS, 1>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
-  return gateup_rows<BITS, 2>(routed, shared, tab_dev, tab_val, n_slots, x, act, st);
+  // Rounds of 5 chunks per lane where they divide the row into fewer places
+  // than rounds of 4 (2560: one of 5, not two of 4).
+  const uint32_t n = (routed.hidden / kChunk + 15) / 16;
+  const bool five = (n + 4) / 5 * 5 < (n + 3) / 4 * 4;
+  auto rows = [&](auto p) {
+    if (n == 1) return fn(p, std::integral_constant<int, 1>{});
+    return five ? fn(p, std::integral_constant<int, 5>{}) : fn(p, std::integral_constant<int, 4>{});
+  };
+  return n_slots * routed.inter <= 4096 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});
+}
+constexpr uint32_t kPhW = 4;  // waves per gate/up block
+static uint32_t ph_tiles(uint32_t inter, uint32_t p) { return (inter + 4 * p * kPhW - 1) / (4 * p * kPhW); }
+static uint32_t ph_x_lds(uint32_t hidden, uint32_t ib) {
+  return (hidden / kChunk + 16 * ib - 1) / (16 * ib) * (16 * ib) * kL4Words * 4;
+}
+
+template <int BITS>
+static hipError_t gateup_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
+                              const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
+  return gateup_shape(routed, n_slots, [&](auto p, auto ib) {
+    constexpr int P = decltype(p)::value, IB = decltype(ib)::value;
+    const uint32_t tiles = ph_tiles(routed.inter, P);
+    hipLaunchKernelGGL((k_ph_gateup<BITS, P, IB, kPhW>), dim3(tiles * n_slots), dim3(64 * kPhW), ph_x_lds(routed.hidden, IB), st,
+                       routed, shared, tab_dev, tab_val, tiles, x, act);
+    return hipGetLastError();
+  });
+}
+
+// Hidden 4096 has gate/up waves of its own (decode.hip); the selection reads
+// eight logits per lane at most.
+bool ph_route_supported(uint32_t hidden, uint32_t n_experts) { return hidden != 4096 && n_experts <= 512; }
+
+template <int BITS, int PL>
+static hipError_t route_bits(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t E,
+                             uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
+                             float* act, hipStream_t st) {
+  return gateup_shape(routed, n_slots, [&](auto p, auto ib) {
+    constexpr int P = decltype(p)::value, IB = decltype(ib)::value;
+    const uint32_t tiles = ph_tiles(routed.inter, P);
+    hipLaunchKernelGGL((k_ph_route<BITS, PL, P, IB, kPhW>), dim3(tiles * n_slots + 1), dim3(64 * kPhW),
+                       ph_x_lds(routed.hidden, IB), st, routed, shared, logits, E, k, (int)normalize, out, tiles, x, act);
+    return hipGetLastError();
+  });
+}
+
+hipError_t launch_ph_route(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t E,
+                           uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
+                           float* act, hipStream_t st) {
+  if (routed.bits == 4)
+    return E <= 256 ? route_bits<4, 4>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st)
+                    : route_bits<4, 8>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st);
+  return E <= 256 ? route_bits<3, 4>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st)
+                  : route_bits<3, 8>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st);
 }
 
 hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
@@ -383,7 +540,8 @@ bool ph_down_supported(uint32_t inter, uint32_t k, bool has_shared) {
 template <int BITS, uint32_t NR, int TB>
 static hipError_t down_inst(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
-                            const float* h_mid, const float* shared_out, float* hidden_out, hipStream_t st) {
+                            const float* h_mid, const float* shared_out, float* hidden_out, bool ordered,
+                            hipStream_t st) {
   const uint32_t lds = ph_down_lds((k + has_shared) * (routed.inter / kChunk), NR);
   if (lds > 60 * 1024) {
     static std::atomic<uint64_t> raised{0};
@@ -392,25 +550,26 @@ static hipError_t down_inst(const BlobGeom& routed, const BlobGeom& shared, cons
   }
   hipLaunchKernelGGL((k_ph_down<BITS, NR, TB>), dim3((routed.hidden + NR - 1) / NR),
                      dim3(64 * ph_down_waves(routed.inter, k, has_shared)), lds, st, routed, shared, tab_dev, tab_val, k,
-                     has_shared, act, h_mid, shared_out, hidden_out);
+                     has_shared, act, h_mid, shared_out, hidden_out, (int)ordered);
   return hipGetLastError();
 }
 
 template <int BITS>
 static hipError_t down_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
-                            const float* h_mid, const float* shared_out, float* hidden_out, hipStream_t st) {
+                            const float* h_mid, const float* shared_out, float* hidden_out, bool ordered,
+                            hipStream_t st) {
   if (ph_down_waves(routed.inter, k, has_shared) <= 8)
-    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
-  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
+    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
+  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
 }
 
 hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                           const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
-                          const float* shared_out, float* hidden_out, hipStream_t st) {
+                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered) {
   const uint32_t k = tab_val.k, has_shared = n_slots > k ? 1u : 0u;
-  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st)
-                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, st);
+  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st)
+                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
 }
 
 }  // namespace smoe
