@@ -34,18 +34,23 @@ struct Limbs4 {
 
 // A chunk's values as limbs, four lanes per chunk (lane q of the quad holds
 // values 8 q .. 8 q + 7): x_j = m_j 2^-f, |m_j| <= 2^30, bytes in the order of
-// unpack_bytes. live: store.
+// unpack_bytes. f <= 149: 2^-f is a float, and at 149 every m_j is exact. A
+// chunk with an infinity: its finite values 0, the infinities +-2^30 at a scale
+// of infinity, so that a product is infinite or NaN as an f32 one is (a NaN
+// comes from the sum xs). live: store.
 __device__ __forceinline__ void store_limbs4_quad(uint32_t* dst, const float (&x)[8], int q, bool live) {
   float amax = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
   amax = fmaxf(amax, dpp_f<0xB1>(amax, 0.f));
   amax = fmaxf(amax, dpp_f<0x4E>(amax, 0.f));
-  const int f = amax > 0.f ? 30 - __builtin_amdgcn_frexp_expf(amax) : 0;
+  const bool inf = amax == INFINITY;
+  const int f = inf ? -200 : amax > 0.f ? min(30 - __builtin_amdgcn_frexp_expf(amax), 149) : 0;
   int32_t d[4][8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const int32_t m = (int32_t)__builtin_rintf(__builtin_ldexpf(x[j], f));
+    const float v = __builtin_amdgcn_fmed3f(__builtin_ldexpf(x[j], f), -0x1p30f, 0x1p30f);
+    const int32_t m = (int32_t)__builtin_rintf(v);
     const int32_t d0 = (int32_t)((uint32_t)m << 24) >> 24, m1 = (m - d0) >> 8;
     const int32_t d1 = (int32_t)((uint32_t)m1 << 24) >> 24, m2 = (m1 - d1) >> 8;
     const int32_t d2 = (int32_t)((uint32_t)m2 << 24) >> 24;
@@ -59,7 +64,7 @@ __device__ __forceinline__ void store_limbs4_quad(uint32_t* dst, const float (&x
   for (int L = 0; L < 4; ++L)
     *reinterpret_cast<uint2*>(dst + 8 * L + 2 * q) = make_uint2(
         pack_bytes(d[L][0], d[L][2], d[L][4], d[L][6]), pack_bytes(d[L][1], d[L][3], d[L][5], d[L][7]));
-  if (q == 0) *reinterpret_cast<uint2*>(dst + 32) = make_uint2(__float_as_uint(__builtin_ldexpf(1.0f, -f)), __float_as_uint(xs));
+  if (q == 0) *reinterpret_cast<uint2*>(dst + 32) = make_uint2(__float_as_uint(inf ? INFINITY : __builtin_ldexpf(1.0f, -f)), __float_as_uint(xs));
 }
 
 __device__ __forceinline__ void load_limbs4(const uint32_t* p, Limbs4& o) {

@@ -6,8 +6,9 @@ oracle's sequential f32 sums of K <= 8128 terms are off by about sqrt(K) 2^-24,
 import numpy as np
 import pytest
 
-from helpers import rel_err
-from test_gpu_decode import _experts_case, _layer_case, _torch
+import oracle
+from helpers import gen_expert_blob, rel_err
+from test_gpu_decode import _experts_case, _layer_case, _torch, dev, host
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +75,36 @@ def test_phase_nonfinite_input(kernels):
     assert kernels.experts_decode(lay, bind, [0.5, 0.5], x, h, None, 0.0, out) == 0
     kernels.sync()
     assert bool(torch.isfinite(out).all())
+
+
+@pytest.mark.parametrize("scale", [1.0, 2e-19, 1e-19])
+def test_phase_range_ends(kernels, scale):
+    """SwiGLU outputs near the smallest normal float keep their precision, and
+    an infinity in the hidden vector reaches every output, zero biases
+    included. Bar 1e-5 as above, and 1152 steps of the smallest subnormal: both
+    sides round 192 SwiGLU outputs (times a weight <= 1.1), 192 products and
+    192 sums by at most one each."""
+    import streamoe_amd as sa
+
+    H, I = 576, 192
+    rng = np.random.default_rng(11)
+    blob = gen_expert_blob(rng, H, I, 64, 4)
+    blob.reshape(3, -1)[:, H * I // 2 + H * I // 32:] = 0
+    lay = sa.ExpertLayout(H, I, 4, 64)
+    arena = dev(blob)
+    x = (rng.standard_normal(H) * scale).astype(np.float32)
+    zero, out = dev(np.zeros(H, np.float32)), dev(np.zeros(H, np.float32))
+
+    def run():
+        assert kernels.experts_decode(lay, [(arena, 0)], [1.0], dev(x), zero, None, 0.0, out) == 0
+        kernels.sync()
+        return host(out)
+
+    want = oracle.expert_swiglu(blob, 4, H, I, 64, x)
+    top = float(np.abs(want).max())
+    got = run()
+    err = float(np.abs(got.astype(np.float64) - want).max()) / top
+    print(f"scale {scale}: largest output {top:.3e}, rel_err={err:.3e}")
+    assert err <= TOL + 1152 * 2.0 ** -149 / top
+    x[100] = np.inf
+    assert not np.isfinite(run()).any()
