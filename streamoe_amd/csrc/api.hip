@@ -544,16 +544,22 @@ static int check_layer(smoe_handle* h, const smoe_layer* L) {
 
 // With norm_w, `input` is the residual: the router kernel normalises it
 // (bf16 weights norm_w, eps) and stores the normalised row in x_norm, which
-// the expert kernels then read.
+// the expert kernels then read. Several tokens (rows of input, h_mid,
+// hidden_out, x_norm, idx_out, w_out) only where phase_tokens_ok.
+static bool phase_tokens_ok(const smoe_layer* L) {
+  return ph_route_supported(L->shape.hidden, L->n_experts) &&
+         ph_down_supported(L->shape.inter, L->k, L->shared_expert != nullptr);
+}
 static int decode_layer(smoe_handle* h, const smoe_layer* L, const float* input,
                         const float* h_mid, float* hidden_out, int32_t* idx_out, float* w_out,
-                        const uint16_t* norm_w = nullptr, float eps = 0.f, float* x_norm = nullptr) {
+                        const uint16_t* norm_w = nullptr, float eps = 0.f, float* x_norm = nullptr,
+                        uint32_t n_tokens = 1) {
   const smoe_expert_shape& s = L->shape;
   Q8Rows rq, gq;
   layer_q8(L, &rq, &gq);
   hipError_t e = launch_router_logits(L->router_w, L->shared_expert ? L->shared_gate : nullptr,
-                                      input, 1, L->n_experts, s.hidden, h->logits, h->gate,
-                                      h->stream, norm_w, eps, x_norm, rq, gq);
+                                      input, n_tokens, L->n_experts, s.hidden, h->logits, h->gate,
+                                      h->stream, norm_w, eps, x_norm, rq, gq, h->lstride);
   if (norm_w) input = x_norm;
   if (e != hipSuccess) return SMOE_ERR_HIP;
   RouteOut ro{};
@@ -569,10 +575,12 @@ static int decode_layer(smoe_handle* h, const smoe_layer* L, const float* input,
   FfnTable tv{};
   tv.k = L->k;
   const uint32_t n_slots = L->k + (L->shared_expert ? 1 : 0);
-  if (ph_route_supported(s.hidden, L->n_experts) && ph_down_supported(s.inter, L->k, n_slots > L->k)) {
-    e = launch_ph_route(g, gs, h->logits, L->n_experts, L->k, L->normalize != 0, ro, n_slots, input, h->act, h->stream);
+  if (phase_tokens_ok(L)) {
+    e = launch_ph_route(g, gs, h->logits, L->n_experts, L->k, L->normalize != 0, ro, n_slots, input, h->act, h->stream,
+                        n_tokens, h->lstride, h->astride);
     if (e != hipSuccess) return SMOE_ERR_HIP;
-    return hip_status(launch_ph_down(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out, h->stream, true));
+    return hip_status(launch_ph_down(g, gs, h->table, tv, n_slots, h->act, h_mid, nullptr, hidden_out, h->stream, true,
+                                     n_tokens, h->astride));
   }
   e = launch_topk(h->logits, 1, L->n_experts, L->k, true, L->normalize != 0, ro, h->stream);
   if (e != hipSuccess) return SMOE_ERR_HIP;
@@ -679,11 +687,11 @@ int smoe_moe_decode_layer(smoe_handle* h, const smoe_layer* layer, const float* 
   return decode_layer(h, layer, input, h_mid, hidden_out, idx_out, w_out);
 }
 
-// One token through the layers on the per-phase kernels (RMSNorm launch,
-// then one layer), with the last layer's idx / w when asked.
+// The layers on the per-phase kernels, one token or (where phase_tokens_ok
+// for every layer) several, with the last layer's idx / w when asked.
 static int decode_chain_phases(smoe_handle* h, const smoe_layer* layers, uint32_t n_layers,
                                const void* const* norm_w, float eps, const float* input, float* residual_io,
-                               float* work, int32_t* idx_out, float* w_out) {
+                               float* work, int32_t* idx_out, float* w_out, uint32_t n_tokens = 1) {
   for (uint32_t l = 0; l < n_layers; ++l) {
     const bool last = l + 1 == n_layers;
     // Layers after the first read the residual; with norm weights their
@@ -691,7 +699,7 @@ static int decode_chain_phases(smoe_handle* h, const smoe_layer* layers, uint32_
     const float* x = l > 0 ? residual_io : input;
     const uint16_t* nw = (l > 0 && norm_w) ? (const uint16_t*)norm_w[l] : nullptr;
     if (int rc = decode_layer(h, &layers[l], x, residual_io, residual_io, last ? idx_out : nullptr,
-                              last ? w_out : nullptr, nw, eps, work))
+                              last ? w_out : nullptr, nw, eps, work, n_tokens))
       return rc;
   }
   return SMOE_OK;
@@ -779,7 +787,12 @@ int smoe_moe_decode_tokens(smoe_handle* h, const smoe_layer* layers, uint32_t n_
   if (int rc = use_device(h)) return rc;
   if (!all) {
     // Shapes without a three-kernel instance (or the per-phase path asked
-    // for): each token through the per-phase chain in turn.
+    // for): the per-phase chain, over all tokens at once where its kernels
+    // have the token axis, else for each token in turn.
+    bool at_once = true;
+    for (uint32_t l = 0; l < n_layers; ++l) at_once = at_once && phase_tokens_ok(&layers[l]);
+    if (at_once)
+      return decode_chain_phases(h, layers, n_layers, norm_w, eps, input, residual_io, work, idx_out, w_out, n_tokens);
     const uint32_t H = layers[0].shape.hidden, K = layers[n_layers - 1].k;
     for (uint32_t t = 0; t < n_tokens; ++t)
       if (int rc = decode_chain_phases(h, layers, n_layers, norm_w, eps, input + (size_t)t * H,

@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256) void k_router_logits(const float* __restrict__
                                                        const float* __restrict__ gate_w,
                                                        const float* __restrict__ x,
                                                        uint32_t n_experts, uint32_t hidden,
-                                                       float* __restrict__ logits,
+                                                       float* __restrict__ logits, uint32_t lstride,
                                                        float* __restrict__ gate_scores,
                                                        const uint16_t* __restrict__ norm_w, float eps,
                                                        float* __restrict__ x_out, Q8Rows Wq, Q8Rows gq) {
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(256) void k_router_logits(const float* __restrict__
   if (threadIdx.x == 0) {
     const float s = (red[0] + red[1]) + (red[2] + red[3]);
     if (e < n_experts)
-      logits[(size_t)t * n_experts + e] = s;
+      logits[(size_t)t * lstride + e] = s;
     else
       gate_scores[t] = s;
   }
@@ -610,10 +610,10 @@ hipError_t launch_router_logits(const float* W, const float* gate_w, const float
                                 uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
                                 float* logits, float* gate_scores, hipStream_t st,
                                 const uint16_t* norm_w, float eps, float* x_out, const Q8Rows& Wq,
-                                const Q8Rows& gq) {
+                                const Q8Rows& gq, uint32_t lstride) {
   const uint32_t rows = n_experts + (gate_w || gq.q ? 1 : 0);
   hipLaunchKernelGGL(k_router_logits, dim3(rows, n_tokens), dim3(256), 0, st, W, gate_w, x,
-                     n_experts, hidden, logits, gate_scores, norm_w, eps, x_out, Wq, gq);
+                     n_experts, hidden, logits, lstride ? lstride : n_experts, gate_scores, norm_w, eps, x_out, Wq, gq);
   return hipGetLastError();
 }
 

@@ -244,7 +244,8 @@ hipError_t launch_router_logits(const float* W, const float* gate_w, const float
                                 uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
                                 float* logits, float* gate_scores, hipStream_t st,
                                 const uint16_t* norm_w = nullptr, float eps = 0.f, float* x_out = nullptr,
-                                const Q8Rows& Wq = Q8Rows{}, const Q8Rows& gq = Q8Rows{});
+                                const Q8Rows& Wq = Q8Rows{}, const Q8Rows& gq = Q8Rows{},
+                                uint32_t lstride = 0);  // floats per token's logits; 0: n_experts
 // The same for many tokens (f32 router, no gate, no norm) on MFMA (router.hip).
 bool router_mm_supported(uint32_t n_tokens, uint32_t n_experts, uint32_t hidden);
 hipError_t launch_router_mm(const float* W, const float* x, uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
@@ -273,16 +274,19 @@ hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared,
 hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st);
 // The routing (from the logits, at least 64 P floats readable, P = 4 or 8) and
-// the gate/up step in one launch; the table's slots are then in its own
-// order, so the down step has to take table.order (ordered).
+// the gate/up step of n_tokens tokens in one launch; a table's slots are then
+// in its own order, so the down step has to take table.order (ordered).
+// Token t: logits + t lstride (a multiple of 4), table + t, x + t hidden,
+// act + t astride, idx and weight + t k, gate_scores + t.
 bool ph_route_supported(uint32_t hidden, uint32_t n_experts);
 hipError_t launch_ph_route(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t n_experts,
                            uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
-                           float* act, hipStream_t st);
+                           float* act, hipStream_t st, uint32_t n_tokens, uint32_t lstride, uint32_t astride);
 bool ph_down_supported(uint32_t inter, uint32_t k, bool has_shared);
 hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                           const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
-                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered = false);
+                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered = false,
+                          uint32_t n_tokens = 1, uint32_t astride = 0);
 // Streaming-read diagnostic over `bytes` (multiple of 16) with
 // kStreamBlocks blocks; sink: kStreamBlocks u32.
 constexpr uint32_t kStreamBlocks = 2048;

@@ -215,6 +215,8 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeo
 // were a launch of their own between the router and the experts (39 -> 32 us
 // per layer at 2560 x 640). It writes the table in the order the
 // act rows have, and the place of each of the reference's slots in it.
+// Grid y: tokens, so that a layer of several is one launch (2560 x 640, 8
+// layers, two / four tokens: 503 / 996 us one after another, 376 / 620 so).
 // ---------------------------------------------------------------------------
 template <int PL>
 struct RouteLds {
@@ -280,14 +282,23 @@ __device__ void ph_route_table(const float* __restrict__ logits, uint32_t E, uin
 template <int BITS, int PL, int P, int IB, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom shared, const float* __restrict__ logits,
                                                        uint32_t E, uint32_t k, int normalize, RouteOut ro, uint32_t tiles,
-                                                       const float* __restrict__ x, float* __restrict__ act) {
+                                                       const float* __restrict__ x, float* __restrict__ act,
+                                                       uint32_t lstride, uint32_t astride) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
   __shared__ RouteLds<PL> rl[WPB];
+  const uint32_t t = blockIdx.y;
+  logits += (size_t)t * lstride;
+  x += (size_t)t * routed.hidden;
+  act += (size_t)t * astride;
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (4 * P);
   // Every wave of a block goes the same way (they read the same logits), so
   // the barriers inside are met by all of them.
   if (blockIdx.x == gridDim.x - 1) {
+    ro.table += t;
+    if (ro.idx) ro.idx += (size_t)t * k;
+    if (ro.weight) ro.weight += (size_t)t * k;
+    if (ro.gate_scores) ro.gate_scores += t;
     ph_route_table<PL>(logits, E, k, normalize, ro, wave, (int)lane, rl[0]);
     return;
   }
@@ -364,8 +375,14 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
                                                   FfnTable tab_val, uint32_t k, uint32_t has_shared,
                                                   const float* __restrict__ act, const float* h_mid,
                                                   const float* __restrict__ shared_out, float* hidden_out,
-                                                  int ordered) {
+                                                  int ordered, uint32_t astride) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  if (tab_dev) {  // grid y: tokens
+    tab_dev += blockIdx.y;
+    act += (size_t)blockIdx.y * astride;
+    h_mid += (size_t)blockIdx.y * routed.hidden;
+    hidden_out += (size_t)blockIdx.y * routed.hidden;
+  }
   __shared__ uint8_t sord[kMaxK];
   __shared__ float so[NR][kMaxSlots + 1];
   __shared__ float sw[kMaxSlots];
@@ -466,7 +483,7 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
 // ---------------------------------------------------------------------------
 // Calls fn with the instance's (P, IB) as integral constants.
 template <typename F>
-static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {
+static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {  // n_slots: of all tokens
   // 4 rows per wave while that makes no more than 1024 waves (one per SIMD),
   // else 8, whose limbs serve two rows each: 8 slots of 2048 x 512 (gate/up
   // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
@@ -507,24 +524,25 @@ bool ph_route_supported(uint32_t hidden, uint32_t n_experts) { return hidden != 
 template <int BITS, int PL>
 static hipError_t route_bits(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t E,
                              uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
-                             float* act, hipStream_t st) {
-  return gateup_shape(routed, n_slots, [&](auto p, auto ib) {
+                             float* act, hipStream_t st, uint32_t n_tokens, uint32_t lstride, uint32_t astride) {
+  return gateup_shape(routed, n_slots * n_tokens, [&](auto p, auto ib) {
     constexpr int P = decltype(p)::value, IB = decltype(ib)::value;
     const uint32_t tiles = ph_tiles(routed.inter, P);
-    hipLaunchKernelGGL((k_ph_route<BITS, PL, P, IB, kPhW>), dim3(tiles * n_slots + 1), dim3(64 * kPhW),
-                       ph_x_lds(routed.hidden, IB), st, routed, shared, logits, E, k, (int)normalize, out, tiles, x, act);
+    hipLaunchKernelGGL((k_ph_route<BITS, PL, P, IB, kPhW>), dim3(tiles * n_slots + 1, n_tokens), dim3(64 * kPhW),
+                       ph_x_lds(routed.hidden, IB), st, routed, shared, logits, E, k, (int)normalize, out, tiles, x, act,
+                       lstride, astride);
     return hipGetLastError();
   });
 }
 
 hipError_t launch_ph_route(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t E,
                            uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
-                           float* act, hipStream_t st) {
-  if (routed.bits == 4)
-    return E <= 256 ? route_bits<4, 4>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st)
-                    : route_bits<4, 8>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st);
-  return E <= 256 ? route_bits<3, 4>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st)
-                  : route_bits<3, 8>(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st);
+                           float* act, hipStream_t st, uint32_t n_tokens, uint32_t lstride, uint32_t astride) {
+  auto go = [&](auto fn) {
+    return fn(routed, shared, logits, E, k, normalize, out, n_slots, x, act, st, n_tokens, lstride, astride);
+  };
+  if (routed.bits == 4) return E <= 256 ? go(route_bits<4, 4>) : go(route_bits<4, 8>);
+  return E <= 256 ? go(route_bits<3, 4>) : go(route_bits<3, 8>);
 }
 
 hipError_t launch_ph_gateup(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
@@ -546,16 +564,16 @@ template <int BITS, uint32_t NR, int TB>
 static hipError_t down_inst(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
                             const float* h_mid, const float* shared_out, float* hidden_out, bool ordered,
-                            hipStream_t st) {
+                            hipStream_t st, uint32_t n_tokens, uint32_t astride) {
   const uint32_t lds = ph_down_lds((k + has_shared) * (routed.inter / kChunk), NR);
   if (lds > 60 * 1024) {
     static std::atomic<uint64_t> raised{0};
     const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(&k_ph_down<BITS, NR, TB>), kPdLds, raised);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_ph_down<BITS, NR, TB>), dim3((routed.hidden + NR - 1) / NR),
+  hipLaunchKernelGGL((k_ph_down<BITS, NR, TB>), dim3((routed.hidden + NR - 1) / NR, n_tokens),
                      dim3(64 * ph_down_waves(routed.inter, k, has_shared)), lds, st, routed, shared, tab_dev, tab_val, k,
-                     has_shared, act, h_mid, shared_out, hidden_out, (int)ordered);
+                     has_shared, act, h_mid, shared_out, hidden_out, (int)ordered, astride);
   return hipGetLastError();
 }
 
@@ -563,18 +581,19 @@ template <int BITS>
 static hipError_t down_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                             const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
                             const float* h_mid, const float* shared_out, float* hidden_out, bool ordered,
-                            hipStream_t st) {
+                            hipStream_t st, uint32_t n_tokens, uint32_t astride) {
   if (ph_down_waves(routed.inter, k, has_shared) <= 8)
-    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
-  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
+    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
+  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
 }
 
 hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                           const FfnTable& tab_val, uint32_t n_slots, const float* act, const float* h_mid,
-                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered) {
+                          const float* shared_out, float* hidden_out, hipStream_t st, bool ordered,
+                          uint32_t n_tokens, uint32_t astride) {
   const uint32_t k = tab_val.k, has_shared = n_slots > k ? 1u : 0u;
-  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st)
-                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st);
+  return routed.bits == 4 ? down_bits<4>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride)
+                          : down_bits<3>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
 }
 
 }  // namespace smoe

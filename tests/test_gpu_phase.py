@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 from helpers import gen_expert_blob, rel_err
-from test_gpu_decode import _experts_case, _layer_case, _torch, dev, host
+from test_gpu_decode import _chain, _experts_case, _layer_case, _torch, dev, host
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +108,36 @@ def test_phase_range_ends(kernels, scale):
     assert err <= TOL + 1152 * 2.0 ** -149 / top
     x[100] = np.inf
     assert not np.isfinite(run()).any()
+
+
+@pytest.mark.parametrize("T,H,I,E,k,bits,norm", [
+    (4, 2560, 640, 64, 10, 4, 0.1),
+    (2, 2048, 640, 41, 3, 3, 0.0),     # odd logit rows
+    (3, 320, 192, 300, 16, 4, 0.1),    # eight logits per lane, most slots
+    (4, 7168, 1920, 18, 8, 4, 0.1),    # two rounds of chunks, down blocks of four rows
+])
+def test_phase_tokens_match_single_token(kernels, T, H, I, E, k, bits, norm):
+    """Several tokens through the per-phase kernels at once: outputs, indices
+    and weights bit for bit those of each token alone."""
+    torch = _torch()
+    kernels.reserve(max(H, 4096), 2048, 1024)
+    c = _chain(kernels, 2, E, k, bits, seed=H + E + T, norm_sigma=norm, I=I, H=H)
+    xs = dev(np.random.default_rng(T).standard_normal((T, H)).astype(np.float32))
+    xs[:, 0] *= 50
+
+    def run(rows):
+        r, n = rows.clone(), rows.shape[0]
+        idx = torch.empty((n, k), dtype=torch.int32, device="cuda")
+        w = torch.empty((n, k), dtype=torch.float32, device="cuda")
+        assert kernels.moe_decode_tokens(c["layers"], c["norms"], 1e-6, n, rows, r, torch.empty_like(rows), idx, w) == 0
+        kernels.sync()
+        return host(r).view(np.uint32), host(idx), host(w).view(np.uint32)
+
+    kernels.set_decode_path(1)
+    try:
+        got = run(xs)
+        one = [run(xs[t:t + 1].contiguous()) for t in range(T)]
+    finally:
+        kernels.set_decode_path(0)
+    for a, b in zip(got, zip(*one)):
+        assert np.array_equal(a, np.concatenate(b))
