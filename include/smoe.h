@@ -406,7 +406,8 @@ int smoe_moe_decode_layers_noalloc(void* stream, const smoe_layer* layers, uint3
  * tokens take a fourth launch per layer (the router kernel in two
  * halves). Shapes without a three-kernel instance (and
  * SMOE_OPT_DECODE_PATH = 1) run the per-phase kernels over all tokens
- * (more than 512 experts, hidden 4096: each token in turn), bit-identical to smoe_moe_decode_layers on that token; with
+ * (more than 512 experts, hidden 4096: each token in turn), a token
+ * bit-identical to smoe_moe_decode_layers on it alone; with
  * SMOE_OPT_DECODE_PATH = 3 they return SMOE_ERR_UNSUPPORTED_SHAPE. */
 int smoe_moe_decode_tokens(smoe_handle* h, const smoe_layer* layers, uint32_t n_layers,
                            const void* const* norm_w, float eps, uint32_t n_tokens, const float* input,
