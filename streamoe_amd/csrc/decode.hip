@@ -642,7 +642,7 @@ __global__ __launch_bounds__(64) void k_topk(const float* __restrict__ scores, u
   }
   if (softmax) {
     // moe_router.rs:52-72, the reference's probabilities bit for bit.
-    __shared__ float sprob[64 * P];
+    __shared__ alignas(16) float sprob[64 * P];
     softmax_ref<P, true>(v, n, lane, sprob, load_exp_tab(lane));
     if (out.probs) {
 #pragma unroll

@@ -504,7 +504,7 @@ __global__ __launch_bounds__(64) void k_fa_gateup(FusedLayer a_all) {
   const FusedLayer a = token_view<HC>(a_all, blockIdx.y);
   __shared__ int32_t sid[kMaxK];
   __shared__ float sval[kMaxK];
-  __shared__ float sprob[64 * P];  // the exact softmax's values (softmax_ref)
+  __shared__ alignas(16) float sprob[64 * P];  // the exact softmax's values (softmax_ref)
   FaClock clk;
   fa_stamp(a, clk, 0, false);
   const int lane = threadIdx.x;

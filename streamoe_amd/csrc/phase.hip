@@ -218,9 +218,11 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeo
 // Grid y: tokens, so that a layer of several is one launch (2560 x 640, 8
 // layers, two / four tokens: 503 / 996 us one after another, 376 / 620 so).
 // ---------------------------------------------------------------------------
+// softmax_ref reads prob in 16-byte pieces, in every element of an array of
+// these (one per wave).
 template <int PL>
 struct RouteLds {
-  float prob[64 * PL];
+  alignas(16) float prob[64 * PL];
   float val[kMaxK];
   int32_t id[kMaxK], set[kMaxK];
   int32_t is_set;
@@ -237,13 +239,13 @@ __device__ void ph_route_table(const float* __restrict__ logits, uint32_t E, uin
     l[e] = jl < E ? logits[jl] : -INFINITY;
   }
   // The set on a wave of its own beside the scan (the other waves only meet
-  // the barriers: three in softmax_ref, one after the scan).
+  // the barriers: those of softmax_ref, and one after the scan).
   if (wave != 0) {
     if (wave == 1) {
       const bool set = topk_set_logits<PL>(l, E, k, lane, s.set);
       if (lane == 0) s.is_set = set;
     }
-    for (int i = 0; i < 4; ++i) __syncthreads();
+    for (int i = 0; i < kSoftmaxBarriers + 1; ++i) __syncthreads();
     return;
   }
   softmax_ref<PL, true>(v, E, lane, s.prob, load_exp_tab(lane));
@@ -286,6 +288,7 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom
                                                        uint32_t lstride, uint32_t astride) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
   __shared__ RouteLds<PL> rl[WPB];
+  static_assert(alignof(RouteLds<PL>) == 16 && sizeof(RouteLds<PL>) % 16 == 0, "rl[wave].prob is read by 16 bytes");
   const uint32_t t = blockIdx.y;
   logits += (size_t)t * lstride;
   x += (size_t)t * routed.hidden;

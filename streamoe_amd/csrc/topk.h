@@ -17,11 +17,15 @@ namespace smoe {
 // lane l owns [l*P, l*P + P) (TR = false) or l, l + 64, ... (TR = true).
 // Positions >= n become -inf. The max is the wave's fmaxf (it differs from
 // the reference's strict-> scan only when a NaN is present, and then every
-// probability is NaN in both). The sum runs over sbuf (LDS, >= 64 P
-// floats, which also receives the probabilities): every lane adds the same
-// broadcast values, so all lanes hold the sum. `tab` is this lane's table
-// entry (load_exp_tab). Single-wave blocks only (one barrier).
+// probability is NaN in both). The sum runs over sbuf (LDS, 64 P floats on a
+// 16-byte boundary, read by 16 bytes; it also receives the probabilities):
+// every lane adds the same broadcast values, so all lanes hold the sum. `tab`
+// is this lane's table entry (load_exp_tab). kSoftmaxBarriers block barriers:
+// every wave of the block has to meet as many, here (with an sbuf of its own)
+// or elsewhere.
 // ---------------------------------------------------------------------------
+constexpr int kSoftmaxBarriers = 3;
+
 struct ExpTabReg {
   uint32_t lo, hi;  // kExpTab[lane & 31]
 };
@@ -58,8 +62,7 @@ __device__ __forceinline__ void softmax_ref(float (&v)[P], uint32_t n, int lane,
   // Sequential sum in index order; the zeros past n change nothing (the sum
   // of non-negative values is never -0). 32 values per round, the next
   // round's LDS reads under way during a round's additions (a read waited for
-  // every four additions cost 1.2 us at 512
-  // experts).
+  // every four additions cost 1.2 us at 512 experts).
   float sum = 0.f;
   const f32x4* s4 = reinterpret_cast<const f32x4*>(sbuf);
   f32x4 cur[8], nxt[8];

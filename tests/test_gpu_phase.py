@@ -9,6 +9,7 @@ import pytest
 import oracle
 from helpers import gen_expert_blob, rel_err
 from test_gpu_decode import _chain, _experts_case, _layer_case, _torch, dev, host
+from test_gpu_softmax import _same_bits as same_bits, ulp_cases
 
 pytestmark = pytest.mark.gpu
 
@@ -141,3 +142,46 @@ def test_phase_tokens_match_single_token(kernels, T, H, I, E, k, bits, norm):
         kernels.set_decode_path(0)
     for a, b in zip(got, zip(*one)):
         assert np.array_equal(a, np.concatenate(b))
+
+
+@pytest.mark.parametrize("E,k", [(256, 8), (257, 16), (300, 4), (512, 10)])
+def test_phase_routing_boundary(kernels, E, k):
+    """Four tokens at once whose k-th and (k+1)-th logits are 0, 1 and 2 ulps
+    apart (every gate/up wave then runs the reference's softmax and scan) beside
+    one with a clear margin: indices and weights bit for bit the oracle's,
+    together and one at a time."""
+    import streamoe_amd as sa
+
+    torch = _torch()
+    H, I, T = 320, 192, 4
+    rng = np.random.default_rng(E + k)
+    cols = ulp_cases(E, k, 3, 60 + E + k) + [rng.standard_normal(E).astype(np.float32)]
+    router = np.zeros((E, H), np.float32)
+    router[:, :T] = np.stack(cols, axis=1)
+    lay = sa.ExpertLayout(H, I, 4, 64)
+    arena = torch.empty(E * lay.expert_size, dtype=torch.uint8, device="cuda")
+    assert kernels.synth_experts(arena, E, lay.expert_size, lay, E) == 0
+    shared = dev(gen_expert_blob(rng, H, I, 64, 4))
+    gate = rng.standard_normal(H).astype(np.float32)
+    router_d, gate_d = dev(router), dev(gate)  # the layer holds their addresses
+    layer = kernels.layer(lay, arena, lay.expert_size, E, k, True, router_d, shared, gate_d)
+    x = np.eye(T, H, dtype=np.float32)
+    want = [oracle.moe_decode_layer(host(arena), lay.expert_size, H, I, E, k, 64, 4, True, router, x[t], x[t],
+                                    host(shared), gate) for t in range(T)]
+    for t in range(T):
+        assert same_bits(want[t][3], cols[t])  # one-hot rows: the logits are the columns
+
+    def run(rows):
+        r, n = dev(rows), len(rows)
+        idx = torch.empty((n, k), dtype=torch.int32, device="cuda")
+        w = torch.empty((n, k), dtype=torch.float32, device="cuda")
+        assert kernels.moe_decode_tokens([layer], None, 1e-6, n, dev(rows), r, torch.empty_like(r), idx, w) == 0
+        kernels.sync()
+        return host(r), host(idx), host(w)
+
+    got = run(x)
+    for t in range(T):
+        out, idx, w = run(x[t:t + 1])
+        assert np.array_equal(got[1][t], want[t][1]) and np.array_equal(idx[0], want[t][1])
+        assert same_bits(got[2][t], want[t][2]) and same_bits(w[0], want[t][2])
+        assert rel_err(got[0][t], want[t][0]) <= TOL and same_bits(out[0], got[0][t])
