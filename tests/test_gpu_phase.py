@@ -30,6 +30,10 @@ TOL = 1e-5
     (128, 2048, 16, 3, True),   # 1024: a wave per row
 ])
 def test_phase_experts_match_oracle(kernels, H, I, k, bits, shared):
+    _check_experts(kernels, H, I, k, bits, shared)
+
+
+def _check_experts(kernels, H, I, k, bits, shared):
     if H > 4096:
         kernels.reserve(H, 2048, 1024)
     got, want, h_mid = _experts_case(kernels, H, I, k, bits, shared, seed=H + I + k + bits)
@@ -185,3 +189,13 @@ def test_phase_routing_boundary(kernels, E, k):
         assert np.array_equal(got[1][t], want[t][1]) and np.array_equal(idx[0], want[t][1])
         assert same_bits(got[2][t], want[t][2]) and same_bits(w[0], want[t][2])
         assert rel_err(got[0][t], want[t][0]) <= TOL and same_bits(out[0], got[0][t])
+
+
+@pytest.mark.parametrize("H,I,k,bits,shared", [
+    # The row's limbs in one to four rounds of a block's threads.
+    (2112, 64, 4, 4, False),    # 66 chunks: two rounds, the second of two
+    (6208, 320, 7, 3, True),    # 194: four
+    (8192, 192, 11, 4, False),  # 256: four whole ones
+])
+def test_phase_long_rows_match_oracle(kernels, H, I, k, bits, shared):
+    _check_experts(kernels, H, I, k, bits, shared)
