@@ -524,12 +524,16 @@ static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {
   // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
   // 2560 x 640 18.8 against 17.3, 8 of 7168 x 2048 74.0 against 72.2. Four
   // waves share a block's limbs (one: 12.2, two: 11.3 at 2048 x 512).
-  // Rounds of 5 chunks per lane where they divide the row into fewer places
+  // Rounds of as many chunks per lane as the row has up to three (1024: rounds
+  // of 4 left half of the places empty, 8 slots of 1024 x 1536 19.7 us against
+  // 15.3), of 5 where they divide the row into fewer places
   // than rounds of 4 (2560: one of 5, not two of 4).
   const uint32_t n = (routed.hidden / kChunk + 15) / 16;
   const bool five = (n + 4) / 5 * 5 < (n + 3) / 4 * 4;
   auto rows = [&](auto p) {
     if (n == 1) return fn(p, std::integral_constant<int, 1>{});
+    if (n == 2) return fn(p, std::integral_constant<int, 2>{});
+    if (n == 3) return fn(p, std::integral_constant<int, 3>{});
     return five ? fn(p, std::integral_constant<int, 5>{}) : fn(p, std::integral_constant<int, 4>{});
   };
   return n_slots * routed.inter <= 4096 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});

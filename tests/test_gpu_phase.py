@@ -199,3 +199,13 @@ def test_phase_routing_boundary(kernels, E, k):
 ])
 def test_phase_long_rows_match_oracle(kernels, H, I, k, bits, shared):
     _check_experts(kernels, H, I, k, bits, shared)
+
+
+@pytest.mark.parametrize("H,I,k,bits,shared", [
+    (576, 64, 1, 4, False),  # 18 chunks: two per lane, most of the second's past the row
+    (1024, 576, 8, 4, True),      # 32: two, 8 rows per wave
+    (1088, 192, 3, 3, False),     # 34: three
+    (1536, 320, 14, 3, True),     # 48: three, 8 rows per wave
+])
+def test_phase_short_rows_match_oracle(kernels, H, I, k, bits, shared):
+    _check_experts(kernels, H, I, k, bits, shared)
