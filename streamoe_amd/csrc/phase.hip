@@ -204,7 +204,11 @@ __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobG
 #pragma unroll
         for (int m = 0; m < 2; ++m)
           sum[p][m] += chunk_dot4<BITS>(raw[i][p][m], xl, __uint_as_float(sv[i][p][m] << 16), __uint_as_float(bv[i][p][m] << 16));
-      __builtin_amdgcn_sched_barrier(0);  // one chunk's limbs in registers at a time
+      // One chunk's limbs in registers at a time: its dots end here, and the
+      // next chunk's reads stay behind them (a scheduling barrier alone left the
+      // dots behind the last read: up to 458 registers, one wave per SIMD).
+#pragma unroll
+      for (int p = 0; p < P; ++p) asm volatile("" : "+v"(sum[p][0]), "+v"(sum[p][1]) : : "memory");
     }
     c0 += 16 * IB;
     if (c0 >= cpr) break;
