@@ -369,7 +369,8 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom
 
 // ---------------------------------------------------------------------------
 // Down + combine. One block per NR hidden rows (8; 4 in blocks of more
-// than 8 waves, whose lanes have half the registers); a lane owns one (slot,
+// than 8 waves, whose lanes have half the registers, and where 8 would leave
+// CUs without a block); a lane owns one (slot,
 // chunk) of the flat list of k * inter / 32 and reads it for all the rows, so only
 // the last wave has empty lanes; one more wave takes the shared expert's
 // chunks (4-bit). The products go to LDS, a thread per (row, slot) adds a
@@ -624,9 +625,14 @@ static hipError_t down_bits(const BlobGeom& routed, const BlobGeom& shared, cons
                             const FfnTable& tab_val, uint32_t k, uint32_t has_shared, const float* act,
                             const float* h_mid, const float* shared_out, float* hidden_out, bool ordered,
                             hipStream_t st, uint32_t n_tokens, uint32_t astride) {
-  if (ph_down_waves(routed.inter, k, has_shared) <= 8)
-    return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
-  return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
+  // Eight rows per block where that still makes a block per CU, else four (8
+  // slots of 1024 x 1536, gate/up and down: 15.1 us with eight, 13.8 with four;
+  // of 512 x 2048 13.8 and 12.3).
+  if (ph_down_waves(routed.inter, k, has_shared) > 8)
+    return down_inst<BITS, 4, 1024>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
+  if ((routed.hidden + 7) / 8 * n_tokens < 256)
+    return down_inst<BITS, 4, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
+  return down_inst<BITS, 8, 512>(routed, shared, tab_dev, tab_val, k, has_shared, act, h_mid, shared_out, hidden_out, ordered, st, n_tokens, astride);
 }
 
 hipError_t launch_ph_down(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,

@@ -209,3 +209,13 @@ def test_phase_long_rows_match_oracle(kernels, H, I, k, bits, shared):
 ])
 def test_phase_short_rows_match_oracle(kernels, H, I, k, bits, shared):
     _check_experts(kernels, H, I, k, bits, shared)
+
+
+@pytest.mark.parametrize("H,I,k,bits,shared", [
+    (1024, 1536, 8, 3, True),    # down blocks of four rows in six waves
+    (1984, 512, 5, 4, False),    # 248 blocks of eight would be fewer than CUs
+    (2048, 512, 5, 4, False),    # 256 are not
+    (64, 2048, 15, 4, False),    # 16 blocks, 15 waves
+])
+def test_phase_down_rows_match_oracle(kernels, H, I, k, bits, shared):
+    _check_experts(kernels, H, I, k, bits, shared)
