@@ -107,11 +107,12 @@ __device__ __forceinline__ const uint8_t* slot_blob(const FfnTable* dev, const F
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up. A wave takes 4 P rows (gate and up) of one slot: 16 lanes per row,
-// lane l the chunks l, l + 16, ..., IB of them per round (the last round's
-// past the row re-read its last chunk against zero limbs). 16 lanes per row
-// leave at most 15 of a row's chunk places empty, where whole-wave rows of
-// 80 chunks left 48 of 128.
+// Gate/up. A wave takes 64 / LR * P rows (gate and up) of one slot: LR lanes
+// per row, lane l the chunks l, l + LR, ..., IB of them per round (the last
+// round's past the row re-read its last chunk against zero limbs). 16 lanes per
+// row, in rounds as long as the row where it has up to 80 chunks, leave at most
+// 15 of its chunk places empty, where whole-wave rows of 80 chunks left 48 of
+// 128; few long rows take 64 (gateup_shape).
 // ---------------------------------------------------------------------------
 // x as limbs: a quad of threads per chunk; chunks past the row are zero. All
 // of a thread's values are loaded at once, ahead of the weights (up to four
@@ -123,10 +124,10 @@ constexpr uint32_t kPhXR = 4;
 constexpr uint32_t kPhNQ = kPhW * kWave / 4;  // chunks per round
 static_assert(kPhXR * kPhNQ * kChunk >= 8192, "the widest row");
 
-template <int IB>
+template <int RC>  // the row is padded to a multiple of RC chunks
 struct StageX {
   f32x4 v[kPhXR][2];
-  static __device__ __forceinline__ uint32_t padded(uint32_t cpr) { return (cpr + 16 * IB - 1) / (16 * IB) * (16 * IB); }
+  static __device__ __forceinline__ uint32_t padded(uint32_t cpr) { return (cpr + RC - 1) / RC * RC; }
   __device__ __forceinline__ void load(const float* x, uint32_t cpr) {
     const uint32_t qd = threadIdx.x >> 2, q = threadIdx.x & 3;
 #pragma unroll
@@ -153,23 +154,23 @@ struct StageX {
 };
 
 // STAGE: the limbs are still to be loaded, and written after the weights' loads.
-template <int BITS, int P, int IB, bool STAGE>
+template <int BITS, int P, int IB, int LR, bool STAGE>
 __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobGeom& g, uint32_t row0, uint32_t lane,
                                                const float* x, uint32_t* limbs, float* act) {
   constexpr int CB = chunk_bytes<BITS>();
   const gbytes blob = as_global(blob_);
   const uint32_t cpr = g.hidden / kChunk, gpr = g.hidden >> __builtin_ctz(g.group);
   const uint32_t cps = __builtin_ctz(g.group / kChunk);
-  const uint32_t l16 = lane & 15, lrow = lane >> 4;
+  const uint32_t lc = lane % LR, lrow = lane / LR;
   uint32_t row[P];
 #pragma unroll
-  for (int p = 0; p < P; ++p) row[p] = min(row0 + p * 4 + lrow, g.inter - 1);
+  for (int p = 0; p < P; ++p) row[p] = min(row0 + p * (64 / LR) + lrow, g.inter - 1);
   Raw<BITS> raw[IB][P][2];
   uint32_t sv[IB][P][2], bv[IB][P][2];
   auto load = [&](uint32_t c0) {
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
-      const uint32_t c = min(c0 + i * 16 + l16, cpr - 1);
+      const uint32_t c = min(c0 + i * LR + lc, cpr - 1);
 #pragma unroll
       for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -181,7 +182,7 @@ __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobG
         }
     }
   };
-  StageX<IB> xs;
+  StageX<IB * LR> xs;
   if constexpr (STAGE) xs.load(x, cpr);
   __builtin_amdgcn_sched_barrier(0);
   load(0);
@@ -198,7 +199,7 @@ __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobG
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
       Limbs4 xl;
-      load_limbs4(limbs + (size_t)(c0 + i * 16 + l16) * kL4Words, xl);
+      load_limbs4(limbs + (size_t)(c0 + i * LR + lc) * kL4Words, xl);
 #pragma unroll
       for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -210,32 +211,33 @@ __device__ __forceinline__ void ph_gateup_rows(const uint8_t* blob_, const BlobG
 #pragma unroll
       for (int p = 0; p < P; ++p) asm volatile("" : "+v"(sum[p][0]), "+v"(sum[p][1]) : : "memory");
     }
-    c0 += 16 * IB;
+    c0 += LR * IB;
     if (c0 >= cpr) break;
     load(c0);
   }
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const float gs = row_sum16_all(sum[p][0]), us = row_sum16_all(sum[p][1]);
-    const uint32_t r = row0 + p * 4 + lrow;
-    if (l16 == 0 && r < g.inter) act[r] = silu_mul(gs, us);
+    const float gs = LR == 16 ? row_sum16_all(sum[p][0]) : group_sum<LR>(sum[p][0]);
+    const float us = LR == 16 ? row_sum16_all(sum[p][1]) : group_sum<LR>(sum[p][1]);
+    const uint32_t r = row0 + p * (64 / LR) + lrow;
+    if (lc == 0 && r < g.inter) act[r] = silu_mul(gs, us);
   }
 }
 
-template <int BITS, int P, int IB, int WPB>
+template <int BITS, int P, int IB, int LR, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeom shared, const FfnTable* __restrict__ tab_dev,
                                                         FfnTable tab_val, uint32_t tiles, const float* __restrict__ x,
                                                         float* __restrict__ act) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (4 * P);
+  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (64 / LR * P);
   const uint32_t k = tab_dev ? tab_dev->k : tab_val.k;
   const uint8_t* const blob = slot_blob(tab_dev, tab_val, slot);
   float* const out = act + (size_t)slot * routed.inter;
   if (slot < k)
-    ph_gateup_rows<BITS, P, IB, true>(blob, routed, row0, lane, x, lds, out);
+    ph_gateup_rows<BITS, P, IB, LR, true>(blob, routed, row0, lane, x, lds, out);
   else
-    ph_gateup_rows<4, P, IB, true>(blob, shared, row0, lane, x, lds, out);
+    ph_gateup_rows<4, P, IB, LR, true>(blob, shared, row0, lane, x, lds, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -314,7 +316,7 @@ __device__ void ph_route_table(const float* __restrict__ logits, uint32_t E, uin
   }
 }
 
-template <int BITS, int PL, int P, int IB, int WPB>
+template <int BITS, int PL, int P, int IB, int LR, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom shared, const float* __restrict__ logits,
                                                        uint32_t E, uint32_t k, int normalize, RouteOut ro, uint32_t tiles,
                                                        const float* __restrict__ x, float* __restrict__ act,
@@ -327,7 +329,7 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom
   x += (size_t)t * routed.hidden;
   act += (size_t)t * astride;
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (4 * P);
+  const uint32_t slot = blockIdx.x / tiles, row0 = (blockIdx.x % tiles * WPB + wave) * (64 / LR * P);
   // Every wave of a block goes the same way (they read the same logits), so
   // the barriers inside are met by all of them.
   if (blockIdx.x == gridDim.x - 1) {
@@ -340,11 +342,11 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom
   }
   float* const out = act + (size_t)slot * routed.inter;
   if (slot == k) {
-    ph_gateup_rows<4, P, IB, true>(ro.shared_blob, shared, row0, lane, x, lds, out);
+    ph_gateup_rows<4, P, IB, LR, true>(ro.shared_blob, shared, row0, lane, x, lds, out);
     return;
   }
   const uint32_t cpr = routed.hidden / kChunk;
-  StageX<IB> xs;
+  StageX<IB * LR> xs;
   xs.load(x, cpr);
   float l[PL];
 #pragma unroll
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_route(BlobGeom routed, BlobGeom
     __syncthreads();
     id = __builtin_amdgcn_readfirstlane(rl[wave].id[slot]);
   }
-  ph_gateup_rows<BITS, P, IB, false>(ro.experts + (uint64_t)id * ro.stride, routed, row0, lane, x, lds, out);
+  ph_gateup_rows<BITS, P, IB, LR, false>(ro.experts + (uint64_t)id * ro.stride, routed, row0, lane, x, lds, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -521,9 +523,21 @@ __global__ __launch_bounds__(TB) void k_ph_down(BlobGeom routed, BlobGeom shared
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
-// Calls fn with the instance's (P, IB) as integral constants.
+// Calls fn with the instance's (P, IB, LR) as integral constants. The sums of
+// a row depend on LR alone, which the number of tokens does not enter.
 template <typename F>
-static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {  // n_slots: of all tokens
+static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, uint32_t n_tokens, F fn) {  // n_slots: of a token
+  const std::integral_constant<int, 16> l16;
+  const uint32_t n = (routed.hidden / kChunk + 15) / 16;
+  // Rows of more chunks than one round of 16 lanes takes, and few of them: a
+  // whole wave per row, which 1 slot of 7168 x 64 (gate/up and down) takes 12.6
+  // us with, 15.2 with 16 lanes; 16 of 7168 x 128 18.1 and 20.0, 16 of 7168 x
+  // 192 22.7 and 22.0.
+  if (n > 5 && n_slots * routed.inter <= 2048) {
+    const std::integral_constant<int, 64> l64;
+    const std::integral_constant<int, 2> p;
+    return n <= 8 ? fn(p, std::integral_constant<int, 2>{}, l64) : fn(p, std::integral_constant<int, 4>{}, l64);
+  }
   // 4 rows per wave while that makes no more than 1024 waves (one per SIMD),
   // else 8, whose limbs serve two rows each: 8 slots of 2048 x 512 (gate/up
   // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
@@ -533,29 +547,29 @@ static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, F fn) {
   // of 4 left half of the places empty, 8 slots of 1024 x 1536 19.7 us against
   // 15.3), of 5 where they divide the row into fewer places
   // than rounds of 4 (2560: one of 5, not two of 4).
-  const uint32_t n = (routed.hidden / kChunk + 15) / 16;
   const bool five = (n + 4) / 5 * 5 < (n + 3) / 4 * 4;
   auto rows = [&](auto p) {
-    if (n == 1) return fn(p, std::integral_constant<int, 1>{});
-    if (n == 2) return fn(p, std::integral_constant<int, 2>{});
-    if (n == 3) return fn(p, std::integral_constant<int, 3>{});
-    return five ? fn(p, std::integral_constant<int, 5>{}) : fn(p, std::integral_constant<int, 4>{});
+    if (n == 1) return fn(p, std::integral_constant<int, 1>{}, l16);
+    if (n == 2) return fn(p, std::integral_constant<int, 2>{}, l16);
+    if (n == 3) return fn(p, std::integral_constant<int, 3>{}, l16);
+    return five ? fn(p, std::integral_constant<int, 5>{}, l16) : fn(p, std::integral_constant<int, 4>{}, l16);
   };
-  return n_slots * routed.inter <= 4096 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});
+  return n_slots * n_tokens * routed.inter <= 4096 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});
 }
-static uint32_t ph_tiles(uint32_t inter, uint32_t p) { return (inter + 4 * p * kPhW - 1) / (4 * p * kPhW); }
-static uint32_t ph_x_lds(uint32_t hidden, uint32_t ib) {
-  return (hidden / kChunk + 16 * ib - 1) / (16 * ib) * (16 * ib) * kL4Words * 4;
+// Blocks per slot, and the bytes of a row's limbs in LDS.
+static uint32_t ph_tiles(uint32_t inter, uint32_t rows) { return (inter + rows * kPhW - 1) / (rows * kPhW); }
+static uint32_t ph_x_lds(uint32_t hidden, uint32_t rc) {
+  return (hidden / kChunk + rc - 1) / rc * rc * kL4Words * 4;
 }
 
 template <int BITS>
 static hipError_t gateup_bits(const BlobGeom& routed, const BlobGeom& shared, const FfnTable* tab_dev,
                               const FfnTable& tab_val, uint32_t n_slots, const float* x, float* act, hipStream_t st) {
-  return gateup_shape(routed, n_slots, [&](auto p, auto ib) {
-    constexpr int P = decltype(p)::value, IB = decltype(ib)::value;
-    const uint32_t tiles = ph_tiles(routed.inter, P);
-    hipLaunchKernelGGL((k_ph_gateup<BITS, P, IB, kPhW>), dim3(tiles * n_slots), dim3(64 * kPhW), ph_x_lds(routed.hidden, IB), st,
-                       routed, shared, tab_dev, tab_val, tiles, x, act);
+  return gateup_shape(routed, n_slots, 1, [&](auto p, auto ib, auto lr) {
+    constexpr int P = decltype(p)::value, IB = decltype(ib)::value, LR = decltype(lr)::value;
+    const uint32_t tiles = ph_tiles(routed.inter, 64 / LR * P);
+    hipLaunchKernelGGL((k_ph_gateup<BITS, P, IB, LR, kPhW>), dim3(tiles * n_slots), dim3(64 * kPhW),
+                       ph_x_lds(routed.hidden, IB * LR), st, routed, shared, tab_dev, tab_val, tiles, x, act);
     return hipGetLastError();
   });
 }
@@ -568,12 +582,12 @@ template <int BITS, int PL>
 static hipError_t route_bits(const BlobGeom& routed, const BlobGeom& shared, const float* logits, uint32_t E,
                              uint32_t k, bool normalize, const RouteOut& out, uint32_t n_slots, const float* x,
                              float* act, hipStream_t st, uint32_t n_tokens, uint32_t lstride, uint32_t astride) {
-  return gateup_shape(routed, n_slots * n_tokens, [&](auto p, auto ib) {
-    constexpr int P = decltype(p)::value, IB = decltype(ib)::value;
-    const uint32_t tiles = ph_tiles(routed.inter, P);
-    hipLaunchKernelGGL((k_ph_route<BITS, PL, P, IB, kPhW>), dim3(tiles * n_slots + 1, n_tokens), dim3(64 * kPhW),
-                       ph_x_lds(routed.hidden, IB), st, routed, shared, logits, E, k, (int)normalize, out, tiles, x, act,
-                       lstride, astride);
+  return gateup_shape(routed, n_slots, n_tokens, [&](auto p, auto ib, auto lr) {
+    constexpr int P = decltype(p)::value, IB = decltype(ib)::value, LR = decltype(lr)::value;
+    const uint32_t tiles = ph_tiles(routed.inter, 64 / LR * P);
+    hipLaunchKernelGGL((k_ph_route<BITS, PL, P, IB, LR, kPhW>), dim3(tiles * n_slots + 1, n_tokens), dim3(64 * kPhW),
+                       ph_x_lds(routed.hidden, IB * LR), st, routed, shared, logits, E, k, (int)normalize, out, tiles, x,
+                       act, lstride, astride);
     return hipGetLastError();
   });
 }

@@ -120,6 +120,9 @@ def test_phase_range_ends(kernels, scale):
     (2, 2048, 640, 41, 3, 3, 0.0),     # odd logit rows
     (3, 320, 192, 300, 16, 4, 0.1),    # eight logits per lane, most slots
     (4, 7168, 1920, 18, 8, 4, 0.1),    # two rounds of chunks, down blocks of four rows
+    (4, 3072, 512, 20, 4, 4, 0.1),     # a wave per gate/up row, 2048 rows of a token
+    (3, 7168, 192, 300, 3, 3, 0.0),    # the same, four chunks per lane
+    (4, 1024, 576, 20, 3, 4, 0.1),     # 4 rows per wave alone, 8 together; down 4 and 8 rows
 ])
 def test_phase_tokens_match_single_token(kernels, T, H, I, E, k, bits, norm):
     """Several tokens through the per-phase kernels at once: outputs, indices
@@ -218,4 +221,15 @@ def test_phase_short_rows_match_oracle(kernels, H, I, k, bits, shared):
     (64, 2048, 15, 4, False),    # 16 blocks, 15 waves
 ])
 def test_phase_down_rows_match_oracle(kernels, H, I, k, bits, shared):
+    _check_experts(kernels, H, I, k, bits, shared)
+
+
+@pytest.mark.parametrize("H,I,k,bits,shared", [
+    (2624, 128, 16, 4, False),  # 2048 rows of 82 chunks: the most that take a wave per row
+    (2624, 192, 11, 4, False),  # 2112: 16 lanes
+    (3648, 64, 1, 3, False),    # 114 chunks
+    (4160, 64, 2, 4, True),     # 130: four per lane, half of the third's past the row
+    (8192, 128, 15, 3, True),   # 256
+])
+def test_phase_wave_per_row_match_oracle(kernels, H, I, k, bits, shared):
     _check_experts(kernels, H, I, k, bits, shared)
