@@ -20,7 +20,11 @@
 // rounds where an f32 sum of the group would, but not within it. The bias
 // term sum_g b_g sum_{j in g} x_j runs on v_mfma_f32_16x16x4_f32 over the
 // group sums (scaled by 2^f), and the result is acc 2^-f. A row with an
-// infinity or NaN gets NaN group sums, so all its outputs are NaN.
+// infinity or NaN gets NaN group sums, so all its outputs are NaN. Groups of 32
+// take v_mfma_i32_16x16x32_i8, one group per operand (masking the other
+// groups' codes to zero in 64-input operands took twice the matrix work, 32
+// mask instructions per tile and step, and registers beyond what there are:
+// 16 rows 2048 -> 152064 115 us against 93).
 #include "common.h"
 #include "kernels.h"
 
@@ -43,8 +47,9 @@ __host__ __device__ constexpr uint32_t lg_gp(uint32_t K, uint32_t G) { return (l
 // inputs of (j, h, kb) are those the lanes kb of k_lg hold as B operand h:
 // for groups of 64, 128 j + 64 h + {0, 32, 16, 48}[kb] (the halves of two
 // lanes' chunks, exchanged by a permlane swap, so that an operand lies in
-// one group); else 128 j + 32 kb + 16 h. Byte order: code words unpack to
-// even codes, then odd codes, of eight.
+// one group); of 32, eight of each of two groups, 128 j + 64 h + 8 kb and 32
+// on (the four lanes' chunks transposed by their words); else 128 j + 32 kb +
+// 16 h. Byte order: code words unpack to even codes, then odd codes, of eight.
 // ---------------------------------------------------------------------------
 template <bool BF16>
 __device__ __forceinline__ void lg_load8(const void* x, uint64_t i, float (&f)[8]) {
@@ -92,20 +97,21 @@ __device__ __forceinline__ void lg_prep_row(const void* x, uint32_t r, uint32_t 
   uint8_t* const lr = limbs + (uint64_t)r * KP * 4;
   for (uint32_t u = lane; u < KP / 16; u += kWave) {  // (j, h, kb) = u / 8, u / 4 % 2, u % 4
     const uint32_t j = u >> 3, h = (u >> 2) & 1, kb = u & 3;
-    const uint32_t pos = G == 64 ? 128 * j + 64 * h + 32 * (kb & 1) + 16 * (kb >> 1) : 128 * j + 32 * kb + 16 * h;
+    // The unit's first and second eight inputs. K is a multiple of 32, so each
+    // eight lies in the row or past it.
+    const uint32_t pos = G == 64   ? 128 * j + 64 * h + 32 * (kb & 1) + 16 * (kb >> 1)
+                         : G == 32 ? 128 * j + 64 * h + 8 * kb
+                                   : 128 * j + 32 * kb + 16 * h;
     float f[16];
-    if (pos < K) {  // K is a multiple of 32: pos + 16 <= K
-      float a[8], b[8];
-      lg_load8<BF16>(x, row + pos, a);
-      lg_load8<BF16>(x, row + pos + 8, b);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) f[i] = a[i], f[8 + i] = b[i];
-    } else {
+    for (uint32_t e = 0; e < 2; ++e) {
+      const uint32_t at = pos + e * (G == 32 ? 32 : 8);
+      float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (at < K) lg_load8<BF16>(x, row + at, a);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) f[i] = 0.f;
+      for (int i = 0; i < 8; ++i) f[8 * e + i] = a[i];
     }
     int32_t d[4][16];
-    float s = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int32_t m = finite ? (int32_t)__builtin_rintf(__builtin_ldexpf(f[i], fx)) : 0;
@@ -114,12 +120,12 @@ __device__ __forceinline__ void lg_prep_row(const void* x, uint32_t r, uint32_t 
       const int32_t d2 = (int32_t)((uint32_t)m2 << 24) >> 24;
       d[0][i] = d0, d[1][i] = d1, d[2][i] = d2, d[3][i] = (m2 - d2) >> 8;
     }
-    // Pairwise sum of the 16 inputs.
-    {
-      float p[8];
+    // Pairwise sums of the two eights.
+    float s[2];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = f[2 * i] + f[2 * i + 1];
-      s = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    for (int e = 0; e < 2; ++e) {
+      const float* const v = f + 8 * e;
+      s[e] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
 #pragma unroll
     for (int L = 0; L < 4; ++L) {
@@ -130,18 +136,18 @@ __device__ __forceinline__ void lg_prep_row(const void* x, uint32_t r, uint32_t 
       v.w = pack_bytes(d[L][9], d[L][11], d[L][13], d[L][15]);
       *reinterpret_cast<u32x4*>(lr + (((uint64_t)j * 2 + h) * 4 + L) * 64 + kb * 16) = v;
     }
-    // Group sums: over kb (G = 64), over h (32), over both (128). KP / 16
-    // is a multiple of 8, so the lanes of a group are active together.
-    if (G == 32) {
-      s += __shfl_xor(s, 4, kWave);
-    } else {
-      s += __shfl_xor(s, 1, kWave);
-      s += __shfl_xor(s, 2, kWave);
-      if (G == 128) s += __shfl_xor(s, 4, kWave);
+    // Group sums: over kb, and over h too with groups of 128. KP / 16 is a
+    // multiple of 8, so the lanes of a group are active together.
+    if constexpr (G != 32) s[0] += s[1];
+#pragma unroll
+    for (int e = 0; e < (G == 32 ? 2 : 1); ++e) {
+      s[e] += __shfl_xor(s[e], 1, kWave);
+      s[e] += __shfl_xor(s[e], 2, kWave);
+      if (G == 128) s[e] += __shfl_xor(s[e], 4, kWave);
+      const bool first = G == 128 ? (u & 7) == 0 : kb == 0;
+      const uint32_t g = G == 32 ? 4 * j + 2 * h + e : G == 64 ? 2 * j + h : j;
+      if (first) xs[g] = finite ? __builtin_ldexpf(s[e], fx) : __builtin_nanf("");
     }
-    const bool first = G == 32 ? h == 0 : G == 64 ? kb == 0 : (u & 7) == 0;
-    const uint32_t g = G == 32 ? 4 * j + kb : G == 64 ? 2 * j + h : j;
-    if (first) xs[g] = finite ? __builtin_ldexpf(s, fx) : __builtin_nanf("");
   }
 }
 
@@ -287,6 +293,20 @@ struct LgArgs {
 
 __device__ __forceinline__ i32x4 mfma_i8(u32x4 a, u32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
+}
+
+// Over 32 inputs: eight of each lane.
+__device__ __forceinline__ i32x4 mfma_i8_32(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, i32x4 c) {
+  return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)a1 << 32) | a0), (long)(((uint64_t)b1 << 32) | b0), c, 0, 0, 0);
+}
+
+// The 4 x 4 words (lane block of 16, register) transposed.
+__device__ __forceinline__ void transpose4(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+  const auto ac = __builtin_amdgcn_permlane32_swap(a, c, false, false);
+  const auto bd = __builtin_amdgcn_permlane32_swap(b, d, false, false);
+  const auto ab = __builtin_amdgcn_permlane16_swap(ac[0], bd[0], false, false);
+  const auto cd = __builtin_amdgcn_permlane16_swap(ac[1], bd[1], false, false);
+  a = ab[0], b = ab[1], c = cd[0], d = cd[1];
 }
 
 // LDS bytes of the scales (or biases) of `rows` weight rows: 16-byte pieces.
@@ -463,6 +483,9 @@ __global__ __launch_bounds__(256, 2) void k_lg(LgArgs a) {
         w.d[i + 2] = r[1];
       }
     }
+    // Word i of the four lanes' chunks (one group each) to lane block i, as
+    // register (group).
+    if constexpr (G == 32 && BITS == 4) transpose4(w.d[0], w.d[1], w.d[2], w.d[3]);
     uint32_t q[8];
     unpack_bytes(w, q);
     if constexpr (G == 64 && BITS == 3) {
@@ -473,23 +496,28 @@ __global__ __launch_bounds__(256, 2) void k_lg(LgArgs a) {
         q[i + 4] = r[1];
       }
     }
+    if constexpr (G == 32 && BITS == 3) {
+      transpose4(q[0], q[2], q[4], q[6]);
+      transpose4(q[1], q[3], q[5], q[7]);
+    }
     b[0] = u32x4{q[0], q[1], q[2], q[3]};
     b[1] = u32x4{q[4], q[5], q[6], q[7]};
   };
-  // The limb sums of group g (of the step's GS) of a tile. Groups of 32:
-  // lane block kb holds group kb, the other lanes' codes enter as zero.
+  // The limb sums of group g (of the step's GS) of a tile.
   auto sums = [&](const u32x4 (&b)[2], uint32_t g, i32x4 (&S)[4]) {
     const i32x4 z = {0, 0, 0, 0};
     if constexpr (G == 64) {
 #pragma unroll
       for (int L = 0; L < 4; ++L) S[L] = mfma_i8(x[g][L], b[g], z);
+    } else if constexpr (G == 32) {
+      const uint32_t h = g / 2, o = g % 2 * 2;
+#pragma unroll
+      for (int L = 0; L < 4; ++L) S[L] = mfma_i8_32(x[h][L][o], x[h][L][o + 1], b[h][o], b[h][o + 1], z);
     } else {
-      const uint32_t keep = G == 128 || kb == g ? 0xFFFFFFFFu : 0u;
-      const u32x4 m0 = b[0] & keep, m1 = b[1] & keep;
 #pragma unroll
-      for (int L = 0; L < 4; ++L) S[L] = mfma_i8(x[0][L], m0, z);
+      for (int L = 0; L < 4; ++L) S[L] = mfma_i8(x[0][L], b[0], z);
 #pragma unroll
-      for (int L = 0; L < 4; ++L) S[L] = mfma_i8(x[1][L], m1, S[L]);
+      for (int L = 0; L < 4; ++L) S[L] = mfma_i8(x[1][L], b[1], S[L]);
     }
   };
   auto fold = [&](const i32x4 (&S)[4], float s, f32x4& acc) {

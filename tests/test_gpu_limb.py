@@ -105,3 +105,27 @@ def test_limb_qmm_matches_oracle(kernels, out_dim, in_dim, group, bits, n):
     assert np.all(np.isfinite(got))
     # The bf16 tiles split x into bf16 pairs: 2^-17 per value.
     assert worst <= (1e-4 if n == 257 else TOL)
+
+
+@pytest.mark.parametrize("out_dim,in_dim,bits,n", [
+    (48, 64, 3, 5),       # two of a step's four groups
+    (100, 160, 4, 9),     # five groups: the second step's first alone
+    (272, 2144, 4, 40),   # 67: 17 steps over four waves, the last of three groups
+    (8300, 224, 3, 33),   # 4 tiles per wave
+    (33000, 480, 4, 18),  # columns split, an odd step
+])
+def test_limb_groups_of_32(kernels, out_dim, in_dim, bits, n):
+    """Outputs that see one group each (all other scales and biases zero): a code
+    or an input in another group's operand shows at full size."""
+    torch = _torch()
+    rng = np.random.default_rng(out_dim + in_dim)
+    codes, s, b = gen_quant_matrix(rng, out_dim, in_dim, 32, bits)
+    keep = np.arange(in_dim // 32) == (np.arange(out_dim) % (in_dim // 32))[:, None]
+    s, b = np.where(keep, s, 0).astype(np.uint16), np.where(keep, b, 0).astype(np.uint16)
+    x = rng.standard_normal((n, in_dim)).astype(np.float32)
+    y = torch.full((n, out_dim), 7.0, dtype=torch.float32, device="cuda")
+    ws = torch.empty(kernels.qmm_workspace_size(in_dim, 32, n), dtype=torch.uint8, device="cuda")
+    assert kernels.qmm(qweights(codes, s, b, 32, bits), dev(x), y, out_dim, in_dim, n, ws) == 0
+    got = host(y)
+    for t in sorted({0, n // 2, n - 1}):
+        assert rel_err(got[t], oracle_matvec(codes, s, b, in_dim, out_dim, 32, bits, x[t])[0]) <= TOL
