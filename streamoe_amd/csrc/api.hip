@@ -315,7 +315,11 @@ int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
     const hipError_t e = launch_qmv(v, x, y, out_dim, in_dim, h->stream, &unsupported);
     if (!unsupported) return hip_status(e);
   }
-  if (limb_ws && limb_qmm_faster(out_dim, in_dim, n_tokens))
+  int n_cu = 0;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess || n_cu <= 0)
+    return SMOE_ERR_HIP;
+  if (limb_ws && limb_qmm_faster(out_dim, in_dim, w->group_size, w->bits, n_tokens,
+                                 qmm_serial_units(out_dim, n_tokens, (uint32_t)n_cu)))
     return hip_status(launch_limb_qmm(v, x, y, out_dim, in_dim, n_tokens, (uint8_t*)workspace, h->stream));
   PfArgs a{};
   qmm_workspace(in_dim, w->group_size, n_tokens, &a, (uint8_t*)workspace);
@@ -331,9 +335,6 @@ int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
   a.n_tokens = n_tokens;
   a.k = 1;
   a.down = y;
-  int n_cu = 0;
-  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess || n_cu <= 0)
-    return SMOE_ERR_HIP;
   return hip_status(launch_qmm(a, x, (uint32_t)n_cu, h->stream));
 }
 

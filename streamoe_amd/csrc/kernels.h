@@ -205,7 +205,7 @@ hipError_t launch_limb_prefill(const BlobGeom& g, const uint8_t* experts, uint64
 // Dense matmul on the same kernel (4- and 3-bit, in_dim a multiple of 32 up
 // to 8192).
 uint64_t limb_qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens);
-bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t n);
+bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group, uint32_t bits, uint32_t n, uint32_t units);
 hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,
                            uint8_t* ws, hipStream_t st);
 bool prefill_supported(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t bits,
@@ -219,6 +219,7 @@ hipError_t launch_prefill(const PfArgs& a, uint32_t n_cu, hipStream_t st);
 // n_tokens, the workspace fields of qmm_workspace, and down = y.
 uint64_t qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens, PfArgs* a, uint8_t* base);
 bool qmm_supported(uint32_t in_dim, uint32_t out_dim, uint32_t group, uint32_t bits, uint32_t n_tokens);
+uint32_t qmm_serial_units(uint32_t out_dim, uint32_t n_tokens, uint32_t n_cu);
 hipError_t launch_qmm(const PfArgs& a, const float* x, uint32_t n_cu, hipStream_t st);
 
 // All launchers return hipSuccess or the launch error; `*unsupported`

@@ -714,17 +714,27 @@ uint64_t limb_qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens) 
 }
 
 // Whether the limb GEMM is the faster one where k_pf_mm has tiles too (at
-// most 8192 inputs). k_pf_mm walks 32-row x 256-column units on one block
-// per CU, each XCD over its own row blocks: a unit's whole K is its latency,
-// and with fewer than 256 rows XCDs stay idle. us, limb against k_pf_mm:
-// 2048 -> 4096 at 16 / 128 / 256 / 512 rows 10.8 / 18.7 / 26.3 / 43.4 against
-// 133 / 48.5 / 28.4 / 30.3; 4096 -> 1024 at 1000 rows 46.9 against 55.4; 512
-// -> 2048 at 256 / 512 rows 10.2 / 13.4 against 11.4 / 12.0; 2048 -> 152064
-// at 128 / 192 rows 334 / 495 against 433 / 432. So: one round of blocks of 8
-// tiles (half a round below 1024 inputs), or up to 128 rows.
-bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t n) {
+// most 8192 inputs). k_pf_mm walks units of 32 rows x 256 columns, the busiest
+// block `units` of them one after another, each with its whole K as latency;
+// the limb GEMM runs rounds of 512 blocks of 16 rows x 128 columns. Measured over
+// 8700 random calls (2 to 1024 rows, 256 to 150000 columns, 256 to 8192 inputs,
+// all groups and bits): where a block has several units, a round of limb blocks
+// per unit is no slower (time against k_pf_mm's 0.5 to 1.09). With one unit it
+// is the faster up to 128 blocks (0.25 to 1.0); up to 256 from 512 inputs on
+// (0.42 to 1.0; 256 inputs, 4 bits 0.9 to 1.15); a whole round (to 512) where a
+// unit costs enough: groups of 64 and 128 from 2048 inputs on (0.66 to 1.09) or,
+// 3 bits, 1024 (0.7 to 0.97), groups of 32 only with 3 bits from 2048 on (0.83
+// to 1.07; 4 bits 0.93 to 1.2); past a round never (1.0 to 2.2). Asking only for
+// 128 rows or one round took one call in twelve over its start, by up to 2.2
+// times (82 rows 2048 -> 16896, group 32: 80 us against 38).
+bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group, uint32_t bits, uint32_t n, uint32_t units) {
   const uint64_t blocks = (uint64_t)((n + kLgM - 1) / kLgM) * ((out_dim + 127) / 128);
-  return in_dim <= 8192 && (n <= 128 || blocks <= (in_dim < 1024 ? kLgRound / 2 : kLgRound));
+  if (in_dim > 8192 || (n > 128 && blocks > (in_dim < 1024 ? kLgRound / 2 : kLgRound))) return false;
+  if (units > 1) return blocks <= (uint64_t)kLgRound * units;
+  const bool large = group > 32, three = bits == 3;
+  if (blocks <= kLgRound / 4) return true;
+  if (blocks <= kLgRound / 2) return in_dim >= 512 || (three && large);
+  return blocks <= kLgRound && (large || three) && in_dim >= (large && three ? 1024u : 2048u);
 }
 
 hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,

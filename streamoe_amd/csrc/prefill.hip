@@ -2573,6 +2573,19 @@ bool qmm_supported(uint32_t in_dim, uint32_t out_dim, uint32_t group, uint32_t b
   return n_tokens >= 1 && n_tokens <= 0xFFFFu - kPfMC;
 }
 
+// The units that the busiest block of launch_qmm's grid walks one after another
+// (k_pf_mm's schedule over row blocks split evenly among the XCDs).
+uint32_t qmm_serial_units(uint32_t out_dim, uint32_t n_tokens, uint32_t n_cu) {
+  const uint64_t nb = (n_tokens + kPfMC - 1) / kPfMC, ncb = out_dim / 256;
+  const uint64_t grid = nb * ncb < n_cu ? nb * ncb : n_cu, nx = grid % 8 == 0 ? 8 : 1, per = grid / nx;
+  uint64_t most = 0;
+  for (uint64_t x = 0; x < nx; ++x) {
+    const uint64_t units = (nb * (x + 1) / nx - nb * x / nx) * ncb;
+    if ((units + per - 1) / per > most) most = (units + per - 1) / per;
+  }
+  return (uint32_t)most;
+}
+
 hipError_t launch_qmm(const PfArgs& a, const float* x, uint32_t n_cu, hipStream_t st) {
   hipLaunchKernelGGL(k_qmm_prep, dim3(a.n_tokens), dim3(256), 0, st, x, a.n_tokens, a.g.inter, a.g.group,
                      a.act_hi, a.act_lo, a.asum, a.items, a.n_items);

@@ -18,8 +18,8 @@ TOL = 1e-3
     (4096, 2048, 32, 4, 33),   # two 32-token blocks
     (1024, 1024, 128, 3, 64),  # packed 3-bit
     (256, 256, 64, 4, 100),    # four blocks, last ragged
-    # Without GEMM tiles (one qmv per token row): Flash-Next's 640 and
-    # 2560, a 7168-wide projection, a 96-input matrix.
+    # Without bf16 GEMM tiles (the limb GEMM): Flash-Next's 640 and 2560, a
+    # 7168-wide projection, a 96-input matrix.
     (640, 2560, 64, 4, 9), (2560, 640, 32, 3, 5), (300, 7168, 64, 4, 3), (64, 96, 32, 4, 17),
 ])
 def test_qmm_matches_oracle(kernels, out_dim, in_dim, group, bits, n):
@@ -56,6 +56,34 @@ def test_qmm_argument_errors(kernels):
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     small = torch.empty(need // 2, dtype=torch.uint8, device="cuda")
     assert kernels.qmm(w, x, y, 512, 2048, 4, small) == c["SMOE_ERR_WORKSPACE_TOO_SMALL"]
-    assert kernels.qmm(w, x, y, 500, 2048, 4, ws) == 0  # out_dim % 256: one qmv per token row
+    assert kernels.qmm(w, x, y, 500, 2048, 4, ws) == 0  # out_dim % 256: the limb GEMM
     assert kernels.qmm(w, x, y, 512, 2048, 0, ws) == c["SMOE_ERR_INVALID_ARG"]
     assert kernels.qmm(w, x[:, 1:], y, 512, 2044, 4, ws) == c["SMOE_ERR_IN_DIM_NOT_MULTIPLE"]
+
+
+@pytest.mark.parametrize("out_dim,in_dim,group,bits,n", [
+    (16896, 2048, 32, 4, 82),    # one unit per block, 792 limb blocks
+    (15104, 4096, 32, 4, 103),
+    (4096, 2048, 32, 4, 256),    # a whole round of limb blocks, group 32
+    (4096, 1024, 64, 4, 256),    # 1024 inputs
+    (1024, 4096, 32, 4, 1000),
+    (5376, 256, 64, 4, 96),      # 252 blocks, 256 inputs
+])
+def test_qmm_stays_on_the_tiles_where_they_are_faster(kernels, out_dim, in_dim, group, bits, n):
+    """Rows of a call that the bf16 tiles take have the same bits within a call
+    of 1024 rows, which they take at any of these shapes."""
+    import torch
+
+    rng = np.random.default_rng(out_dim + n)
+    w = qweights(*gen_quant_matrix(rng, out_dim, in_dim, group, bits), group, bits)
+    x = dev(rng.standard_normal((1024, in_dim)).astype(np.float32))
+
+    def run(rows):
+        y = torch.empty((rows, out_dim), dtype=torch.float32, device="cuda")
+        ws = torch.empty(kernels.qmm_workspace_size(in_dim, group, rows), dtype=torch.uint8, device="cuda")
+        assert kernels.qmm(w, x, y, out_dim, in_dim, rows, ws) == 0
+        return y
+
+    few, many = run(n), run(1024)
+    torch.cuda.synchronize()
+    assert torch.equal(few, many[:n])
