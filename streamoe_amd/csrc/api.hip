@@ -283,12 +283,13 @@ int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, u
   const bool limb_ws = aligned(workspace, 0, 256) && workspace_bytes >= limb_qmm_workspace(in_dim, w->group_size, n_tokens);
   if (!qmm_supported(in_dim, out_dim, w->group_size, w->bits, n_tokens)) {
     // Shapes without bf16 GEMM tiles (in_dim or out_dim not a multiple of
-    // 256, in_dim up to 8192): the limb GEMM; one row, 8-bit weights or a
-    // small workspace: one k_qmv per token row, as smoe_qmv computes it.
+    // 256, in_dim up to 8192): the limb GEMM; one row, two where that is
+    // faster, 8-bit weights or a small workspace: one k_qmv per token row, as
+    // smoe_qmv computes it.
     if (in_dim > 8192) return SMOE_ERR_UNSUPPORTED_SHAPE;
     if (!aligned(x, 0, 16)) return SMOE_ERR_MISALIGNED;
     if (int rc = use_device(h)) return rc;
-    if (n_tokens > 1 && w->bits != 8 && limb_ws)
+    if (n_tokens > 1 && w->bits != 8 && limb_ws && !(n_tokens == 2 && qmm_two_rows_faster(out_dim, in_dim, w->group_size)))
       return hip_status(launch_limb_qmm(v, x, y, out_dim, in_dim, n_tokens, (uint8_t*)workspace, h->stream));
     for (uint32_t t = 0; t < n_tokens; ++t) {
       bool unsupported = false;

@@ -206,6 +206,7 @@ hipError_t launch_limb_prefill(const BlobGeom& g, const uint8_t* experts, uint64
 // to 8192).
 uint64_t limb_qmm_workspace(uint32_t in_dim, uint32_t group, uint32_t n_tokens);
 bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group, uint32_t bits, uint32_t n, uint32_t units);
+bool qmm_two_rows_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group);
 hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,
                            uint8_t* ws, hipStream_t st);
 bool prefill_supported(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t bits,

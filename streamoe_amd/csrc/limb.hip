@@ -737,6 +737,19 @@ bool limb_qmm_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group, uint32_t
   return blocks <= kLgRound && (large || three) && in_dim >= (large && three ? 1024u : 2048u);
 }
 
+// Whether two rows of a shape without tiles are faster on k_qmv, one after the
+// other (three or more never were: 1.05 to 3.8 times the limb GEMM's time).
+// Time of two k_qmv calls against it, group 32: up to 4096 columns 0.73 to 0.97
+// where k_qmv's lanes are mostly full (1056 to 4096 inputs, from 5664 on), 1.09
+// to 1.3 up to 1024 inputs, 1.1 for 4128 to 5600; from 4096 to 16384 columns 1.0
+// to 2.6; wider, up to 2048 inputs, 0.83 to 0.97 (1056 on, or 160 on past 32768
+// columns: 0.82 to 0.98), else 0.9 to 1.7. Groups of 64 and 128: 0.9 to 0.98 at
+// 1056 to 2048 inputs and up to 4096 columns, 0.97 to 3 elsewhere.
+bool qmm_two_rows_faster(uint32_t out_dim, uint32_t in_dim, uint32_t group) {
+  if (out_dim <= 4096) return in_dim > 1024 && (in_dim <= 2048 || (group == 32 && (in_dim <= 4096 || in_dim > 5632)));
+  return group == 32 && out_dim > 16384 && in_dim <= 2048 && in_dim > (out_dim > 32768 ? 128u : 1024u);
+}
+
 hipError_t launch_limb_qmm(const QView& w, const float* x, float* y, uint32_t out_dim, uint32_t in_dim, uint32_t n,
                            uint8_t* ws, hipStream_t st) {
   LgRows r;

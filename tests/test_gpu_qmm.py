@@ -87,3 +87,26 @@ def test_qmm_stays_on_the_tiles_where_they_are_faster(kernels, out_dim, in_dim, 
     few, many = run(n), run(1024)
     torch.cuda.synchronize()
     assert torch.equal(few, many[:n])
+
+
+@pytest.mark.parametrize("out_dim,in_dim,group,bits,n,room", [
+    (300, 7168, 32, 4, 2, "all"),      # two rows that are faster one after the other
+    (640, 1152, 64, 3, 2, "all"),
+    (17000, 1536, 32, 4, 2, "all"),
+    (300, 704, 64, 4, 5, "one byte"),  # a workspace too small for the limb GEMM
+    (300, 704, 64, 3, 5, "unaligned"),
+])
+def test_qmm_row_by_row_is_qmv(kernels, out_dim, in_dim, group, bits, n, room):
+    import torch
+
+    rng = np.random.default_rng(out_dim + in_dim + n)
+    w = qweights(*gen_quant_matrix(rng, out_dim, in_dim, group, bits), group, bits)
+    x = dev(rng.standard_normal((n, in_dim)).astype(np.float32))
+    y, rows = (torch.zeros((n, out_dim), dtype=torch.float32, device="cuda") for _ in range(2))
+    ws = torch.empty(kernels.qmm_workspace_size(in_dim, group, n) + 16, dtype=torch.uint8, device="cuda")
+    ws = {"all": ws, "one byte": ws[:1], "unaligned": ws[16:]}[room]
+    assert kernels.qmm(w, x, y, out_dim, in_dim, n, ws) == 0
+    for t in range(n):
+        assert kernels.qmv(w, x[t], rows[t], out_dim, in_dim) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y, rows)
