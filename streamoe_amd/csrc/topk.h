@@ -265,81 +265,6 @@ __device__ __forceinline__ uint32_t wave_or_last(uint32_t v) {
   return v;
 }
 
-// Top-k SET: the k largest values (ascending index order in set_ids) when
-// the k-th and (k+1)-th largest differ, no value is NaN and the k-th is
-// above the -1e30 start value of the reference's slots. Otherwise returns
-// false and the caller falls back to exact_topk.
-template <int P>
-__device__ bool topk_set(const float (&v)[P], uint32_t n, uint32_t k, int lane,
-                         int32_t* set_ids) {
-  // Each lane sorts its P values descending (stable: lower index first).
-  float sv[P];
-  int32_t si[P];
-#pragma unroll
-  for (int e = 0; e < P; ++e) {
-    sv[e] = v[e];
-    si[e] = lane * P + e;
-  }
-  bool nan = false;
-#pragma unroll
-  for (int e = 0; e < P; ++e) nan |= (sv[e] != sv[e]);
-  if (__ballot(nan)) return false;
-#pragma unroll
-  for (int a = 0; a < P; ++a)
-#pragma unroll
-    for (int b = P - 1; b > a; --b)
-      if (sv[b] > sv[b - 1]) {
-        const float tv = sv[b];
-        sv[b] = sv[b - 1];
-        sv[b - 1] = tv;
-        const int32_t ti = si[b];
-        si[b] = si[b - 1];
-        si[b - 1] = ti;
-      }
-  float kth = 0.f, next = -INFINITY;
-  int taken = 0;  // how many of this lane's sorted values are taken
-  for (uint32_t r = 0; r <= k; ++r) {
-    const float head = taken < P ? sv[0] : -INFINITY;
-    const float m = readlane_f(wave_max_last(head), 63);
-    if (r == k) {
-      next = m;
-      break;
-    }
-    kth = m;
-    const uint64_t ball = __ballot(taken < P && head == m);
-    const int first = __ffsll((unsigned long long)ball) - 1;
-    if (lane == first) {
-#pragma unroll
-      for (int e = 0; e < P - 1; ++e) {
-        sv[e] = sv[e + 1];
-        si[e] = si[e + 1];
-      }
-      sv[P - 1] = -INFINITY;
-      ++taken;
-    }
-  }
-  if (!(kth > next) || !(kth > -1e30f)) return false;
-  // Set = { j : v_j >= kth } (exactly k elements). Compact in index order.
-  int cnt = 0;
-#pragma unroll
-  for (int e = 0; e < P; ++e) cnt += ((uint32_t)(lane * P + e) < n && v[e] >= kth) ? 1 : 0;
-  // Exclusive prefix of cnt over lanes.
-  int incl = cnt;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
-  int at = incl - cnt;
-#pragma unroll
-  for (int e = 0; e < P; ++e) {
-    const uint32_t j = lane * P + e;
-    if (j < n && v[e] >= kth) set_ids[at++] = (int32_t)j;
-  }
-  return true;
-}
-
-
 // ---------------------------------------------------------------------------
 // Top-k SET straight from the logits, for the routed expert kernels.
 //
