@@ -214,24 +214,28 @@ hipError_t launch_noaux_topk(const float* logits, const float* bias, uint32_t n_
 // so the loop has no block barrier. 16-byte part p of row r is stored at part
 // p ^ (r / 4 % 4): the 16 rows of an operand read fall on all banks.
 //
-// Rounding: an accumulator runs over 8 inputs (two MFMAs) and the sums are
-// then added pairwise (a binary tree over a wave's inputs, then over the
-// waves), as the one-row kernel's lanes are, not along one chain of `hidden`
-// additions.
+// Rounding: the sums are those of k_router_logits bit for bit, so a token's
+// logits, and the pick between nearly tied experts, do not depend on how many
+// tokens share the call. Its thread t of 256 chains FMAs over the inputs 1024 i +
+// 4 t + {0, 1, 2, 3}, which is one MFMA per i (the instruction adds its four
+// products one FMA after another); the 256 leaves are then added as a binary
+// tree. Wave w takes the leaves 8 (w + 8 q) .. + 7, q = 0 .. 3, i innermost.
 //
 // 512 tokens, 256 experts, hidden 2048: 94 us with a block per (token, expert
-// row), each reading both rows again (2 GB through L2); 12.4 us
+// row), each reading both rows again (2 GB through L2); 12.5 us
 // here, the limit of its chain of eight pieces per wave (the matrix cores are
 // busy 3.5 us of it).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kRlT = 16, kRlE = 32, kRlW = 8;           // tokens, experts, waves per block
-constexpr uint32_t kRlK = 32;                                // inputs per piece
+constexpr uint32_t kRlK = 32;                                // inputs per piece: eight leaves
+constexpr uint32_t kRlTurn = 1024;                           // inputs from one FMA group of a leaf to the next
+constexpr uint32_t kRlQ = kRlTurn / kRlK / kRlW;             // leaf groups per wave
 constexpr uint32_t kRlRows = kRlT + kRlE;                    // rows of a piece
 constexpr uint32_t kRlPiece = kRlRows * kRlK * 4;            // bytes
 constexpr uint32_t kRlRing = 2;                              // pieces in LDS per wave
 constexpr uint32_t kRlLds = kRlW * kRlRing * kRlPiece;
 static_assert(kRlLds <= 160 * 1024, "LDS per CU");
-static_assert(kRlLds >= kRlW * 2 * 64 * 16, "the waves' sums fit over the pieces");
+static_assert(kRlLds >= (kRlW * kRlQ + kRlQ) * 2 * 64 * 16, "the groups' sums fit over the pieces");
 
 __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict__ W, const float* __restrict__ x,
                                                          uint32_t n, uint32_t E, uint32_t H,
@@ -249,84 +253,85 @@ __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict
   src[0] = reinterpret_cast<const uint8_t*>(x + (size_t)min(t0 + lr, n - 1) * H) + part;
   src[1] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + lr, E - 1) * H) + part;
   src[2] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + 16 + lr, E - 1) * H) + part;
-  // Piece i of this wave: inputs [32 (wave + 8 i), + 32), as two 16-input
-  // columns of 64 bytes per row.
+  // Piece (q, i): inputs [1024 i + 32 (wave + 8 q), + 32), as two 16-input
+  // columns of 64 bytes per row. Group q has `turns(q)` of them.
   constexpr uint32_t NC = kRlK / 16;
-  const uint32_t np = (H / kRlK + kRlW - 1 - wave) / kRlW;
-  auto copy = [&](uint32_t i) {
-    const uint32_t k0 = (wave + kRlW * i) * (kRlK * 4);
-    uint8_t* const dst = mine + i % kRlRing * kRlPiece;
+  auto turns = [&](uint32_t q) {
+    const uint32_t at = (wave + kRlW * q) * kRlK;
+    return at < H ? (H - at + kRlTurn - 1) / kRlTurn : 0u;
+  };
+  uint32_t issued = 0;  // pieces copied so far
+  auto copy = [&](uint32_t q, uint32_t i) {
+    const uint32_t k0 = (i * kRlTurn + (wave + kRlW * q) * kRlK) * 4;
+    uint8_t* const dst = mine + issued++ % kRlRing * kRlPiece;
 #pragma unroll
     for (uint32_t g = 0; g < 3; ++g)
 #pragma unroll
       for (uint32_t c = 0; c < NC; ++c) dma16(src[g] + k0 + c * 64, dst + (g * NC + c) * 1024);
   };
-  f32x4 sum[2][8];  // pairwise tree of each tile: level v holds 2^v pieces' sums
-  uint32_t have = 0;
-  if (np) copy(0);
-  const uint32_t rd = c16 * 64 + ((kb ^ (c16 >> 2)) * 16);  // operand part of lane (row, kb)
-  for (uint32_t i = 0; i < np; ++i) {
-    // The reads of the piece before are done, its buffer takes the next
-    // piece's copies; then this piece has landed when this wave's copies of
-    // it have (the next piece's six stay in flight; a third buffer 13.0 us).
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (i + 1 < np) {
-      copy(i + 1);
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    const uint8_t* const p = mine + i % kRlRing * kRlPiece + rd;
-    static_assert(3 * NC == 6, "copies per piece");
-    f32x4 leaf[2][2 * NC];
+  // Lane (row, kb)'s input 4 m + kb of a column.
+  uint32_t rd[4];
 #pragma unroll
-    for (uint32_t c = 0; c < NC; ++c) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(p + c * 1024);
+  for (uint32_t m = 0; m < 4; ++m) rd[m] = c16 * 64 + ((m ^ (c16 >> 2)) * 16) + kb * 4;
+  f32x4 sum[kRlQ][2];
+  uint32_t done = 0;
+  if (turns(0)) copy(0, 0);
 #pragma unroll
-      for (uint32_t t = 0; t < 2; ++t) {
-        const f32x4 b = *reinterpret_cast<const f32x4*>(p + ((t + 1) * NC + c) * 1024);
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        leaf[t][2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, z, 0, 0, 0);
-        leaf[t][2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, z, 0, 0, 0);
-        leaf[t][2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, leaf[t][2 * c], 0, 0, 0);
-        leaf[t][2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, leaf[t][2 * c + 1], 0, 0, 0);
-      }
-    }
-    f32x4 s[2];
+  for (uint32_t q = 0; q < kRlQ; ++q) {
+    f32x4 leaf[2][4 * NC];
 #pragma unroll
-    for (uint32_t t = 0; t < 2; ++t) s[t] = (leaf[t][0] + leaf[t][1]) + (leaf[t][2] + leaf[t][3]);
-    // Binary counter: carry the sum up past the levels that are full.
-    bool done = false;
-#pragma unroll
-    for (uint32_t v = 0; v < 8; ++v) {
-      if (done) continue;
-      if (have >> v & 1) {
-        s[0] += sum[0][v];
-        s[1] += sum[1][v];
+    for (uint32_t m = 0; m < 4 * NC; ++m) leaf[0][m] = leaf[1][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t ni = turns(q);
+    for (uint32_t i = 0; i < ni; ++i) {
+      // The reads of the piece before are done, its buffer takes the next
+      // piece's copies; then this piece has landed when this wave's copies of
+      // it have (the next piece's six stay in flight; a third buffer 13.0 us).
+      // Later groups have no more turns than this one.
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const bool here = i + 1 < ni, next = q + 1 < kRlQ && turns(q + 1) > 0;
+      if (here || next) {
+        copy(here ? q : q + 1, here ? i + 1 : 0);
+        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
       } else {
-        sum[0][v] = s[0];
-        sum[1][v] = s[1];
-        done = true;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
-    }
-    ++have;
-  }
-  f32x4 tot[2] = {};
+      static_assert(3 * NC == 6, "copies per piece");
+      const uint8_t* const p = mine + done++ % kRlRing * kRlPiece;
+      auto word = [&](uint32_t g, uint32_t c, uint32_t m) {
+        return *reinterpret_cast<const float*>(p + rd[m] + (g * NC + c) * 1024);
+      };
 #pragma unroll
-  for (uint32_t v = 0; v < 8; ++v)
-    if (have >> v & 1) {
-      tot[0] += sum[0][v];
-      tot[1] += sum[1][v];
+      for (uint32_t c = 0; c < NC; ++c)
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m) {
+          const float a = word(0, c, m);
+#pragma unroll
+          for (uint32_t t = 0; t < 2; ++t)
+            leaf[t][4 * c + m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, word(t + 1, c, m), leaf[t][4 * c + m], 0, 0, 0);
+        }
     }
-  // The waves' sums, pairwise.
+#pragma unroll
+    for (uint32_t t = 0; t < 2; ++t)
+      sum[q][t] = ((leaf[t][0] + leaf[t][1]) + (leaf[t][2] + leaf[t][3])) + ((leaf[t][4] + leaf[t][5]) + (leaf[t][6] + leaf[t][7]));
+  }
+  // The tree over the 32 groups, group w + 8 q from wave w: eight groups of one
+  // tile by each wave, then the four sums.
   __syncthreads();
   f32x4* const red = reinterpret_cast<f32x4*>(lds);
-  red[(wave * 2 + 0) * 64 + lane] = tot[0];
-  red[(wave * 2 + 1) * 64 + lane] = tot[1];
+#pragma unroll
+  for (uint32_t q = 0; q < kRlQ; ++q)
+#pragma unroll
+    for (uint32_t t = 0; t < 2; ++t) red[((wave + kRlW * q) * 2 + t) * 64 + lane] = sum[q][t];
+  __syncthreads();
+  {
+    const f32x4* const p = red + (wave >> 1) * 8 * 128 + (wave & 1) * 64 + lane;
+    const f32x4 v = ((p[0] + p[128]) + (p[256] + p[384])) + ((p[512] + p[640]) + (p[768] + p[896]));
+    red[kRlW * kRlQ * 128 + wave * 64 + lane] = v;
+  }
   __syncthreads();
   if (wave < 2) {
-    const f32x4* const p = red + wave * 64 + lane;
-    const f32x4 v = ((p[0] + p[128]) + (p[256] + p[384])) + ((p[512] + p[640]) + (p[768] + p[896]));
+    const f32x4* const p = red + kRlW * kRlQ * 128 + wave * 64 + lane;
+    const f32x4 v = (p[0] + p[128]) + (p[256] + p[384]);
     const uint32_t e = e0 + wave * 16 + c16;
     if (e < E)
 #pragma unroll
@@ -337,13 +342,12 @@ __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict
   }
 }
 
-// Whether a call runs on k_router_mm: whole pieces, no more of them per wave
-// than the tree has room for, and enough logits: a wave's chain of pieces costs
+// Whether a call runs on k_router_mm: whole pieces, and enough logits: a wave's chain of pieces costs
 // 7 us more than one row's block at hidden 2048 (23 at 7168), the one-row
 // kernel 0.27 us per million products, so the line is at about 2^14 logits
 // whatever the hidden size.
 bool router_mm_supported(uint32_t n_tokens, uint32_t n_experts, uint32_t hidden) {
-  return (uint64_t)n_tokens * n_experts >= (1u << 14) && hidden % kRlK == 0 && hidden <= 32768;
+  return (uint64_t)n_tokens * n_experts >= (1u << 14) && hidden % kRlK == 0;
 }
 
 hipError_t launch_router_mm(const float* W, const float* x, uint32_t n_tokens, uint32_t n_experts, uint32_t hidden,
