@@ -185,11 +185,16 @@ uint64_t smoe_qmm_workspace_size(uint32_t in_dim, uint32_t group, uint32_t n_tok
  * biases, x, y 16-byte aligned, biases after the scales; workspace
  * 256-byte aligned. Few rows, small products and the other shapes with
  * in_dim <= 8192 (a multiple of the group; x rows 16-byte aligned) run on
- * int8 MFMA over the rows as 31-bit block floating point (f32 precision; a
- * row with a NaN or an infinity gives a row of NaN). For those other
- * shapes, one row, 8-bit weights and a workspace smaller than
- * smoe_qmm_workspace_size or not 256-byte aligned run smoe_qmv's kernel
- * once per row. Enqueue-only, allocates nothing. */
+ * int8 MFMA over the rows as 31-bit block floating point: one exponent per
+ * row, so an input is off by at most 2^-30 of the row's largest |x| (nothing
+ * from 2^-6 of it up, where f32 keeps no more bits), the sums are f32; a row
+ * with a NaN or an infinity gives a row of NaN. One row, two rows of some of
+ * those other shapes, and for them 8-bit weights or a workspace smaller than
+ * smoe_qmm_workspace_size or not 256-byte aligned run smoe_qmv's kernel row
+ * by row. Which kernel runs, and with fewer than 1024 inputs the order of its
+ * sums, depends on n_tokens, so a row's last bits may differ between calls
+ * of different n_tokens.
+ * Enqueue-only, allocates nothing. */
 int smoe_qmm(smoe_handle* h, const smoe_qweights* w, const float* x, float* y, uint32_t out_dim,
              uint32_t in_dim, uint32_t n_tokens, void* workspace, uint64_t workspace_bytes);
 
@@ -213,7 +218,8 @@ int smoe_dequant(smoe_handle* h, const smoe_qweights* w, uint32_t in_dim, uint32
  * renormalisation when `normalize` (norm_topk_prob).
  * x: device f32[n_tokens, hidden]; idx: device int32[n_tokens, k];
  * weights: device f32[n_tokens, k]; logits_out: device
- * f32[n_tokens, n_experts] or NULL.
+ * f32[n_tokens, n_experts] or NULL. A token's logits are the same bits
+ * whatever n_tokens.
  * Replaces the router gate matvec (attn/linear_attn_forward.rs:2093)
  * plus moe_router_cpu_with (moe_router.rs:165-181) on the host, or on
  * the GPU moe_softmax_topk + moe_normalize_weights (shaders.metal:
@@ -406,7 +412,9 @@ int smoe_moe_decode_layers_noalloc(void* stream, const smoe_layer* layers, uint3
  * tokens take a fourth launch per layer (the router kernel in two
  * halves). Shapes without a three-kernel instance (and
  * SMOE_OPT_DECODE_PATH = 1) run the per-phase kernels over all tokens
- * (more than 512 experts, hidden 4096: each token in turn), a token
+ * (more than 512 experts, hidden 4096, or a layer whose k + shared slots of
+ * inter / 32 chunks exceed a down block, 16 slots of 2048 or 17 from 1888 on:
+ * each token in turn), a token
  * bit-identical to smoe_moe_decode_layers on it alone; with
  * SMOE_OPT_DECODE_PATH = 3 they return SMOE_ERR_UNSUPPORTED_SHAPE. */
 int smoe_moe_decode_tokens(smoe_handle* h, const smoe_layer* layers, uint32_t n_layers,
@@ -436,9 +444,11 @@ uint64_t smoe_moe_prefill_workspace_size(const smoe_expert_shape* shape, uint32_
  * multiples of 256 with hidden >= 1024, <= 512 experts; every other
  * expert shape of the decode entry points (hidden <= 8192, inter <= 2048,
  * multiples of the group) and more experts run grouped GEMMs on int8 MFMA
- * over the rows as 31-bit block floating point (f32 activations and f32
- * precision throughout; a row with a NaN or an infinity gives NaN for its
- * token; the combine again in ascending expert order). One or two tokens
+ * over the rows as 31-bit block floating point (f32 activations and sums;
+ * an input or SwiGLU output is off by at most 2^-30 of its row's largest
+ * magnitude, nothing from 2^-6 of it up; a row with a NaN or an infinity
+ * gives NaN for its token; the combine again in ascending expert order; a
+ * token's last bits may differ between calls of different n_tokens). One or two tokens
  * of those, and calls whose workspace is smaller than
  * smoe_moe_prefill_workspace_size but holds one token's intermediates, go
  * one token at a time through the per-phase decode kernels. 1..1024 tokens, 1 <= k <= min(16,

@@ -1,5 +1,5 @@
 // limb.hip — quantized GEMMs over f32 activations on the int8 matrix cores
-// (gfx950), for many rows at f32 precision.
+// (gfx950), for many rows.
 //
 //   k_lg_prep     rows (f32 or bf16) -> 31-bit block floating point, one
 //                 exponent per row, as four int8 limbs in the MFMA order,
@@ -11,10 +11,11 @@
 //   k_lg_combine  out[t] = sum over t's entries in ascending expert order
 //                 of fma(down[entry], w[entry], out).
 //
-// The arithmetic: a row is written as x_j = m_j 2^-f with |m_j| < 2^30 and
+// The arithmetic: a row is written as x_j = m_j 2^-f with |m_j| <= 2^30 and
 // m = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3 (signed bytes), so a value keeps its
-// 24 mantissa bits down to 2^-6 of the row's largest and an absolute error
-// of 2^-31 of it below. Codes enter as bytes; the sums of a group,
+// 24 mantissa bits down to 2^-6 of the row's largest and is off by at most
+// 2^-30 of that below: less than f32 rounds the sums by, unless the largest
+// meets a weight of zero. Codes enter as bytes; the sums of a group,
 // S_L = sum_j q_j d_Lj, are exact int32 (|S_L| <= 128 * 15 * 128), and
 //     t = (S0 + 2^8 S1) + 2^16 (S2 + 2^8 S3),  acc = fma(s, t, acc)
 // rounds where an f32 sum of the group would, but not within it. The bias

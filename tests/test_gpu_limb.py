@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import gen_quant_matrix, rel_err
+from helpers import dequant_f64, gen_quant_matrix, rel_err
 from test_gpu_decode import dev, oracle_matvec, qweights
 from test_gpu_prefill import _case, _torch, host
 
@@ -129,3 +129,39 @@ def test_limb_groups_of_32(kernels, out_dim, in_dim, bits, n):
     got = host(y)
     for t in sorted({0, n // 2, n - 1}):
         assert rel_err(got[t], oracle_matvec(codes, s, b, in_dim, out_dim, 32, bits, x[t])[0]) <= TOL
+
+
+def test_limb_outlier_bound(kernels):
+    """One exponent per row: a large input moves the others by up to 2^-30 of it
+    each, which shows where its own weight is zero (even outputs here, their
+    group's bias and its code zero). Bound, output by output: that times the sum
+    of s q + |b|, and 64 roundings of f32 partial sums (11 groups in two sums of
+    two roundings each, the bias chain, four K shares). The other rows keep
+    theirs."""
+    torch = _torch()
+    out_dim, in_dim, n, at, big = 300, 704, 5, 5, 1e6
+    rng = np.random.default_rng(21)
+    codes, s, b = gen_quant_matrix(rng, out_dim, in_dim, 64, 4)
+    codes[::2, at // 2] &= 0x0F  # input 5: the high nibble of byte 2
+    b[::2, 0] = 0
+    x = rng.standard_normal((n, in_dim)).astype(np.float32)
+    x[2, at] = big
+    y = torch.empty((n, out_dim), dtype=torch.float32, device="cuda")
+    ws = torch.empty(kernels.qmm_workspace_size(in_dim, 64, n), dtype=torch.uint8, device="cuda")
+    assert kernels.qmm(qweights(codes, s, b, 64, 4), dev(x), y, out_dim, in_dim, n, ws) == 0
+    got = host(y).astype(np.float64)
+    words = np.ascontiguousarray(codes).view(np.uint32)
+    w = dequant_f64(words, s, b, in_dim, out_dim, 64)
+    parts = dequant_f64(words, s & 0x7FFF, b & 0x7FFF, in_dim, out_dim, 64)  # s q + |b|
+    want = x.astype(np.float64) @ w.T
+    assert np.all(w[::2, at] == 0)
+    parts[::2, at] = 0
+    size = parts @ np.abs(x[2].astype(np.float64))
+    bound = 2.0 ** -30 * big * parts.sum(axis=1) + 64 * 2.0 ** -24 * size
+    err = np.abs(got[2] - want[2])
+    print(f"outlier {big:g}: zero-weight outputs off by {(err / bound)[::2].max():.2f} of the bound, "
+          f"{(err / np.abs(want[2]).max())[::2].max():.1e} of the largest output")
+    assert np.all(err[::2] <= bound[::2])
+    assert rel_err(got[2][1::2], want[2][1::2]) <= TOL
+    for t in (0, 1, 3, 4):
+        assert rel_err(got[t], want[t]) <= TOL
