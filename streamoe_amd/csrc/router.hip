@@ -342,10 +342,10 @@ __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict
   }
 }
 
-// Whether a call runs on k_router_mm: whole pieces, and enough logits: a wave's chain of pieces costs
-// 7 us more than one row's block at hidden 2048 (23 at 7168), the one-row
-// kernel 0.27 us per million products, so the line is at about 2^14 logits
-// whatever the hidden size.
+// Whether a call runs on k_router_mm: whole pieces, and enough logits: a
+// wave's chain of pieces costs 7 us more than one row's block at hidden 2048
+// (21 at 7168), the one-row kernel 0.27 us per million products, so the line is
+// at about 2^14 logits whatever the hidden size.
 bool router_mm_supported(uint32_t n_tokens, uint32_t n_experts, uint32_t hidden) {
   return (uint64_t)n_tokens * n_experts >= (1u << 14) && hidden % kRlK == 0;
 }

@@ -110,3 +110,31 @@ def test_qmm_row_by_row_is_qmv(kernels, out_dim, in_dim, group, bits, n, room):
         assert kernels.qmv(w, x[t], rows[t], out_dim, in_dim) == 0
     torch.cuda.synchronize()
     assert torch.equal(y, rows)
+
+
+@pytest.mark.parametrize("out_dim,in_dim,group,bits,n", [
+    (4096, 2048, 32, 4, 257),   # one row past eight blocks of 32
+    (4096, 2048, 32, 3, 300),
+    (4096, 2048, 64, 3, 515),   # 17 blocks, the last of three rows
+    (4096, 2048, 64, 4, 515),
+    (4096, 2048, 128, 4, 300),
+    (4096, 2048, 128, 3, 257),
+    (256, 8448, 128, 4, 40),    # past the limb GEMM's 8192 inputs
+    (512, 16384, 128, 3, 70),   # the most
+])
+def test_qmm_bf16_tiles_match_oracle(kernels, out_dim, in_dim, group, bits, n):
+    """Calls that the bf16 tiles take. Bar 1e-4: x as bf16 pairs is off by 2^-17
+    per value, whose sum over 2048 inputs and more stays below 2e-5 of the
+    largest output."""
+    import torch
+
+    rng = np.random.default_rng(in_dim + 7 * n + group + bits)
+    codes, s, b = gen_quant_matrix(rng, out_dim, in_dim, group, bits)
+    x = rng.standard_normal((n, in_dim)).astype(np.float32)
+    y = torch.full((n, out_dim), 7.0, dtype=torch.float32, device="cuda")
+    ws = torch.empty(kernels.qmm_workspace_size(in_dim, group, n), dtype=torch.uint8, device="cuda")
+    assert kernels.qmm(qweights(codes, s, b, group, bits), dev(x), y, out_dim, in_dim, n, ws) == 0
+    got = host(y)
+    assert np.all(np.isfinite(got))
+    for t in sorted({0, 31, 32, n // 2, n - 1, min(n - 1, 255), min(n - 1, 256)}):
+        assert rel_err(got[t], oracle_matvec(codes, s, b, in_dim, out_dim, group, bits, x[t])[0]) <= 1e-4
