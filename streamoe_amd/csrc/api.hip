@@ -847,11 +847,12 @@ int smoe_moe_prefill(smoe_handle* h, const smoe_expert_shape* shape, const void*
     return SMOE_ERR_MISALIGNED;
   if (!prefill_supported(shape->hidden, shape->inter, shape->group, shape->bits, n_tokens, n_experts, k)) {
     // Shapes without bf16 / fp16 grouped-GEMM tiles: grouped on the int8
-    // matrix cores from three tokens on; fewer (2560 x 640, top-10: one 21 us
-    // against 46, two 41 against 48, three 61 against 53; 2048 x 512, top-8:
-    // two 27 against 41, three 41 against 34), or a workspace too small for
+    // matrix cores from three tokens on; fewer, or a workspace too small for
     // the grouped call, one token at a time through the per-phase decode
-    // kernels.
+    // kernels (2560 x 640, top-10: one 23 us against 46, two 42 against 48,
+    // three 59 against 55; 2048 x 512, top-8: two 29 against 41, three 42
+    // against 36; three of group 32: 60 against 74, 205 against 350 at 7168 x
+    // 2048, top-8, where one after another took 398 with the float kernels).
     if (n_tokens > 2 &&
         workspace_bytes >= limb_prefill_workspace(shape->hidden, shape->inter, shape->group, n_tokens, n_experts, k)) {
       if (int rc = use_device(h)) return rc;

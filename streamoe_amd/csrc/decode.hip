@@ -733,10 +733,11 @@ hipError_t launch_topk(const float* scores, uint32_t n_tokens, uint32_t n, uint3
 // Fused gate/up + SwiGLU at hidden 4096: one wave per 2 rows (gate and up) of
 // one slot, a whole wave per row, two chunks per lane; the block index
 // enumerates (slot, row pair), slots 0..k-1 routed, slot k the shared
-// expert. Every other width, and every call's down rows, run in phase.hip: at
-// this one, whole waves per row and x in registers are the faster (gate/up
-// and down, 512 experts, top-10, inter 1024: 31 us against 34 with 16 lanes
-// per row).
+// expert. Every other width, and every call's down rows, run in phase.hip. At
+// this one whole waves per row and x in registers were the faster (gate/up and
+// down, 512 experts, top-10, inter 1024: 31 us against 34); since phase.hip
+// loads a row's values at once its kernels are no slower here (10 slots of
+// 4096 x 1024 34.2 us with this one and 32.7, 4-bit; 8 of 512 18.6 and 15.8).
 // ---------------------------------------------------------------------------
 constexpr int kGuChunks = 128, kGuCPL = kGuChunks / kWave, kGuRows = 2;
 
@@ -821,8 +822,8 @@ hipError_t launch_gateup(const BlobGeom& routed, const BlobGeom& shared, const F
 }
 
 // ---------------------------------------------------------------------------
-// Down + combine where (slots, chunks) exceed a block's LDS in phase.hip
-// (inter > 1920 with 15 or 16 slots). One wave = one output row; it loads
+// Down + combine where (slots, chunks) exceed a block's waves or LDS in
+// phase.hip (ph_down_supported: 16 slots of inter 2048, 17 from 1888 on). One wave = one output row; it loads
 // every slot's chunk of those rows up front, then reduces slot by slot in
 // the reference's order: moe = fma(out_k, w_k, moe) (deferred.rs:458-466),
 // then the shared term and the residual.
@@ -931,7 +932,8 @@ hipError_t launch_down_combine(const BlobGeom& routed, const BlobGeom& shared, c
 // have no tiles for (hidden or inter not a multiple of 256, hidden below
 // 1024): per token, a route table of its k experts in ascending expert
 // order (the order moe_permute_fuse_cpu, moe_cpu.rs:282-339, adds them in),
-// then k_gateup and k_down_combine over that table with a zero residual.
+// then the one-token gate/up and down kernels (launch_gateup and
+// launch_down_combine choose them) over that table with a zero residual.
 // ---------------------------------------------------------------------------
 // One wave: token t's table. An expert id out of range or repeated within
 // the token sets the device error word (as the grouped path's bucketing

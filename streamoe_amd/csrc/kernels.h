@@ -194,8 +194,8 @@ uint64_t prefill_tokens_workspace(uint32_t hidden, uint32_t inter, uint32_t n_to
 hipError_t launch_prefill_tokens(const BlobGeom& g, const uint8_t* experts, uint64_t stride, uint32_t E,
                                  const int32_t* idx, const float* w, const void* x, bool x_bf16, uint32_t n,
                                  uint32_t k, float* out, uint8_t* ws, uint32_t* err, hipStream_t st);
-// Prefill on the int8 matrix cores at f32 precision (limb.hip), for the same
-// shapes: every group size, hidden and inter multiples of 32, n * k entries
+// Prefill on the int8 matrix cores, rows in 31 bits under one exponent each
+// (limb.hip), for the same shapes: every group size, hidden and inter multiples of 32, n * k entries
 // up to 65535.
 uint64_t limb_prefill_workspace(uint32_t hidden, uint32_t inter, uint32_t group, uint32_t n_tokens,
                                 uint32_t n_experts, uint32_t k);

@@ -271,8 +271,9 @@ __global__ __launch_bounds__(256) void k_lg_prep(LgRoute rt, uint32_t nb_route, 
 // What bounds it: the fold of the limb sums (24 VALU instructions per tile
 // and group of 64, 33 with the unpacking, against 4 MFMAs) and, with two
 // waves per SIMD, what a unit spends before its first step. 512 tokens,
-// 2560 x 640, 512 experts, top-10 (654 items of 16 rows): gate/up 335 us,
-// down 172 us; the VALU is busy half of that, HBM reads run at 2.5 TB/s.
+// 2560 x 640, 512 experts, top-10 (654 items of 16 rows), traced: gate/up 326 us
+// (305 at least), down 170 (161); counters: VALU busy 57 % and 51 %, matrix
+// cores 23 % and 22 %; HBM reads run at 2.5 TB/s.
 // Steps, gate/up us: operand-order loads (64 cache accesses per load instead
 // of 16) 455; memory-order loads and a lane permute 367; the next group's
 // MFMAs ahead of a fold, one set of weight registers re-filled tile by tile

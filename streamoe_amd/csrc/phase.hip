@@ -10,13 +10,15 @@
 // in LDS as 31-bit block floating point, one exponent per 32 values, in four
 // int8 limbs, written once per block while the weights are in flight: a
 // code then costs one byte unpack and four v_dot4c_i32_i8 per four inputs,
-// the sums are exact, and a chunk is rounded once, at f32 precision.
-// Converting codes to floats for FMAs, with every wave loading the
-// activations again, took 11.4 + 21.6 us per layer at 2560 x 640 (512 experts,
-// top-10, shared expert) and 6.4 + 8.7 at 2048 x 512 top-8; these take 10.5 +
-// 12.2 and 5.8 + 6.4: a launch, the table's and the rows' round trips and the
-// dots after them, at an eighth (2048 x 512) to half (7168 x 2048) of the HBM
-// rate.
+// the sums of a chunk's limbs are exact and a chunk is rounded once, to f32. A
+// value is off by at most 2^-31 of its chunk's power of two (2^-30 of the
+// largest of its 32), and keeps its 24 bits down to 2^-6 of that.
+// Traced per launch, 2560 x 640 (512 experts, top-10, shared expert): 13.4 us
+// with the routing in the launch + 12.4; 2048 x 512 top-8: 5.1 + 6.6.
+// Converting codes to floats for FMAs, with every wave loading the activations
+// again, took 11.4 + 21.6 (and a routing launch of 11) and 6.4 + 8.7. What is
+// left is a launch, the table's and the rows' round trips and the dots after
+// them, at an eighth (2048 x 512) to half (7168 x 2048) of the HBM rate.
 #include <type_traits>
 
 #include "common.h"
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(64 * WPB) void k_ph_gateup(BlobGeom routed, BlobGeo
 // per layer at 2560 x 640). It writes the table in the order the
 // act rows have, and the place of each of the reference's slots in it.
 // Grid y: tokens, so that a layer of several is one launch (2560 x 640, 8
-// layers, two / four tokens: 503 / 996 us one after another, 376 / 620 so).
+// layers, two / four tokens: 503 / 996 us one after another, 320 / 520 so).
 // ---------------------------------------------------------------------------
 // softmax_ref reads prob in 16-byte pieces, in every element of an array of
 // these (one per wave).
@@ -541,8 +543,10 @@ static hipError_t gateup_shape(const BlobGeom& routed, uint32_t n_slots, uint32_
   // 4 rows per wave while that makes no more than 1024 waves (one per SIMD),
   // else 8, whose limbs serve two rows each: 8 slots of 2048 x 512 (gate/up
   // and down) 10.8 us against 11.8, 8 of 2048 x 1024 15.9 against 14.3, 10 of
-  // 2560 x 640 18.8 against 17.3, 8 of 7168 x 2048 74.0 against 72.2. Four
-  // waves share a block's limbs (one: 12.2, two: 11.3 at 2048 x 512).
+  // 2560 x 640 18.8 against 17.3, 8 of 7168 x 2048 74.0 against 72.2 (all four
+  // with the row's values staged one round trip after another; as it is the
+  // faster side takes 10.9, 14.5, 17.4 and 64.3). Four waves share a block's
+  // limbs (one: 12.2, two: 11.3 at 2048 x 512).
   // Rounds of as many chunks per lane as the row has up to three (1024: rounds
   // of 4 left half of the places empty, 8 slots of 1024 x 1536 19.7 us against
   // 15.3), of 5 where they divide the row into fewer places
