@@ -219,10 +219,12 @@ hipError_t launch_noaux_topk(const float* logits, const float* bias, uint32_t n_
 // tokens share the call. Its thread t of 256 chains FMAs over the inputs 1024 i +
 // 4 t + {0, 1, 2, 3}, which is one MFMA per i (the instruction adds its four
 // products one FMA after another); the 256 leaves are then added as a binary
-// tree. Wave w takes the leaves 8 (w + 8 q) .. + 7, q = 0 .. 3, i innermost.
+// tree. Wave w takes the leaves' groups of eight 2 w, 2 w + 1 and 16 above
+// them, i innermost: neighbours meet in its registers, and rows that are not
+// whole turns of 1024 still split evenly (hidden 512 or 2560).
 //
 // 512 tokens, 256 experts, hidden 2048: 94 us with a block per (token, expert
-// row), each reading both rows again (2 GB through L2); 12.5 us
+// row), each reading both rows again (2 GB through L2); 12.1 us
 // here, the limit of its chain of eight pieces per wave (the matrix cores are
 // busy 3.5 us of it).
 // ---------------------------------------------------------------------------
@@ -235,7 +237,8 @@ constexpr uint32_t kRlPiece = kRlRows * kRlK * 4;            // bytes
 constexpr uint32_t kRlRing = 2;                              // pieces in LDS per wave
 constexpr uint32_t kRlLds = kRlW * kRlRing * kRlPiece;
 static_assert(kRlLds <= 160 * 1024, "LDS per CU");
-static_assert(kRlLds >= (kRlW * kRlQ + kRlQ) * 2 * 64 * 16, "the groups' sums fit over the pieces");
+static_assert(kRlQ == 4 && kRlT * kRlE == 64 * kRlW, "pairs of groups; a thread per logit");
+static_assert(kRlLds >= kRlW * 2 * 2 * 64 * 16, "the pairs' sums fit over the pieces");
 
 __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict__ W, const float* __restrict__ x,
                                                          uint32_t n, uint32_t E, uint32_t H,
@@ -253,16 +256,14 @@ __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict
   src[0] = reinterpret_cast<const uint8_t*>(x + (size_t)min(t0 + lr, n - 1) * H) + part;
   src[1] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + lr, E - 1) * H) + part;
   src[2] = reinterpret_cast<const uint8_t*>(W + (size_t)min(e0 + 16 + lr, E - 1) * H) + part;
-  // Piece (q, i): inputs [1024 i + 32 (wave + 8 q), + 32), as two 16-input
-  // columns of 64 bytes per row. Group q has `turns(q)` of them.
+  // Piece (q, i): inputs [1024 i + at(q), + 32), as two 16-input columns of 64
+  // bytes per row. Group q has `turns(q)` of them.
   constexpr uint32_t NC = kRlK / 16;
-  auto turns = [&](uint32_t q) {
-    const uint32_t at = (wave + kRlW * q) * kRlK;
-    return at < H ? (H - at + kRlTurn - 1) / kRlTurn : 0u;
-  };
+  auto at = [&](uint32_t q) { return (2 * wave + (q & 1) + 2 * kRlW * (q >> 1)) * kRlK; };
+  auto turns = [&](uint32_t q) { return at(q) < H ? (H - at(q) + kRlTurn - 1) / kRlTurn : 0u; };
   uint32_t issued = 0;  // pieces copied so far
   auto copy = [&](uint32_t q, uint32_t i) {
-    const uint32_t k0 = (i * kRlTurn + (wave + kRlW * q) * kRlK) * 4;
+    const uint32_t k0 = (i * kRlTurn + at(q)) * 4;
     uint8_t* const dst = mine + issued++ % kRlRing * kRlPiece;
 #pragma unroll
     for (uint32_t g = 0; g < 3; ++g)
@@ -314,32 +315,25 @@ __global__ __launch_bounds__(64 * kRlW) void k_router_mm(const float* __restrict
     for (uint32_t t = 0; t < 2; ++t)
       sum[q][t] = ((leaf[t][0] + leaf[t][1]) + (leaf[t][2] + leaf[t][3])) + ((leaf[t][4] + leaf[t][5]) + (leaf[t][6] + leaf[t][7]));
   }
-  // The tree over the 32 groups, group w + 8 q from wave w: eight groups of one
-  // tile by each wave, then the four sums.
+  // The tree over the 16 pairs of groups, pairs w and w + 8 from wave w: thread
+  // (tile, word) adds that word of each pair's 256 and stores its logit.
   __syncthreads();
-  f32x4* const red = reinterpret_cast<f32x4*>(lds);
 #pragma unroll
-  for (uint32_t q = 0; q < kRlQ; ++q)
+  for (uint32_t j = 0; j < 2; ++j)
 #pragma unroll
-    for (uint32_t t = 0; t < 2; ++t) red[((wave + kRlW * q) * 2 + t) * 64 + lane] = sum[q][t];
+    for (uint32_t t = 0; t < 2; ++t)
+      reinterpret_cast<f32x4*>(lds)[((wave + kRlW * j) * 2 + t) * 64 + lane] = sum[2 * j][t] + sum[2 * j + 1][t];
   __syncthreads();
-  {
-    const f32x4* const p = red + (wave >> 1) * 8 * 128 + (wave & 1) * 64 + lane;
-    const f32x4 v = ((p[0] + p[128]) + (p[256] + p[384])) + ((p[512] + p[640]) + (p[768] + p[896]));
-    red[kRlW * kRlQ * 128 + wave * 64 + lane] = v;
-  }
-  __syncthreads();
-  if (wave < 2) {
-    const f32x4* const p = red + kRlW * kRlQ * 128 + wave * 64 + lane;
-    const f32x4 v = (p[0] + p[128]) + (p[256] + p[384]);
-    const uint32_t e = e0 + wave * 16 + c16;
-    if (e < E)
+  const float* const red = reinterpret_cast<const float*>(lds) + threadIdx.x;
+  float v[16];
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t t = t0 + kb * 4 + i;
-        if (t < n) logits[(size_t)t * E + e] = v[i];
-      }
-  }
+  for (uint32_t j = 0; j < 16; ++j) v[j] = red[j * 512];
+#pragma unroll
+  for (uint32_t d = 1; d < 16; d *= 2)
+#pragma unroll
+    for (uint32_t j = 0; j < 16; j += 2 * d) v[j] += v[j + d];
+  const uint32_t t = t0 + (wave & 3) * 4 + (lane & 3), e = e0 + (wave >> 2) * 16 + (lane >> 2);
+  if (t < n && e < E) logits[(size_t)t * E + e] = v[0];
 }
 
 // Whether a call runs on k_router_mm: whole pieces, and enough logits: a
