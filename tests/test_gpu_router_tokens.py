@@ -33,8 +33,8 @@ def test_router_many_tokens(kernels, n, E, H):
     kernels.sync()
     assert torch.equal(idx, idx2) and torch.equal(w, w2)
     want = x.astype(np.float64) @ W.astype(np.float64).T
-    # Rounding of chains of 8 products and log2(H / 8) <= 13 pairwise levels,
-    # 2^-24 of the partial sums each, which sum |w x| bounds.
+    # Rounding of chains of 4 products per 1024 inputs (12 at most here) and 8
+    # pairwise levels, 2^-24 of the partial sums each, which sum |w x| bounds.
     bound = 21 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T)
     assert np.all(np.abs(lg.cpu().numpy() - want) <= bound)
 
